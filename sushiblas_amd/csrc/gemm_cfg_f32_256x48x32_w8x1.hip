@@ -1,9 +1,8 @@
-// gemm_cfg_f32_256x48x32_w8x1.hip -- instantiates the float 256x64x32 MFMA tile
-// computing its first 48 columns (waves 8x1, prefetch depth 2, 2 wave(s) per
-// SIMD, v_mfma_f32_16x16x4_f32), for 32 < N <= 48.
-#include "launch_mfma_impl.hpp"
+// gemm_cfg_f32_256x48x32_w8x1.hip -- instantiates the fp32 split tile
+// (gemm_split.hpp): 8 waves of 32x48: the 256x64 tile computing its first 48
+// columns.  The name is the plan's (kCfg).
+#include "launch_split_impl.hpp"
 
 namespace sbx {
-template hipError_t launch_mfma<float, 256, 64, 32, 8, 1, 2, 2, 1, 48>(
-    const GemmArgs<float>&, bool, bool, int, hipStream_t);
+template hipError_t launch_split<256, 64, 8, 1, 2, 2, 48>(const GemmArgs<float>&, bool, bool, int, hipStream_t);
 }  // namespace sbx

@@ -330,6 +330,34 @@ __device__ inline void tile_coords(const GemmArgs<T>& p, int id, int& tm, int& t
     else { tm = c; tn = r; }
 }
 
+// What a workgroup computes: a whole tile, or one k-part of a tail tile
+// (blocks [0, num_full) own whole tiles; the rest are (tile, k-part) units).
+// Whole tiles are renumbered so that consecutive ids land on one XCD.
+struct TileUnit {
+    int id, part;
+    bool is_split;
+    int tm, tn;
+};
+
+template <typename T>
+__device__ inline TileUnit tile_unit(const GemmArgs<T>& p)
+{
+    TileUnit t;
+    t.id = blockIdx.x;
+    t.part = 0;
+    t.is_split = t.id >= p.num_full;
+    if (t.is_split) {
+        const int u = t.id - p.num_full;
+        t.id = p.num_full + u / p.split;
+        t.part = u - (u / p.split) * p.split;
+    } else if ((p.num_full & 7) == 0) {
+        const int per_xcd = p.num_full >> 3;
+        t.id = (t.id & 7) * per_xcd + (t.id >> 3);
+    }
+    tile_coords(p, t.id, t.tm, t.tn);
+    return t;
+}
+
 // The reference's ReLU: x > 0 ? x : 0 (NaN and -0 become +0).
 template <typename T>
 __device__ inline T relu_of(T x)
@@ -572,6 +600,153 @@ struct CVec<double, 2> {
 template <int N>
 using Int = std::integral_constant<int, N>;
 
+// ---------------------------------------------------------------------------
+// Epilogue of one tile: a wave's accumulators, C = alpha*acc + beta*C, or a
+// split unit's raw partial.  MapA, MapB: block and slot -> row and column of
+// the wave's tile; MapB::U consecutive blocks hold consecutive columns.
+// ---------------------------------------------------------------------------
+template <typename T, typename MF, typename MapA, typename MapB, int BM, int BN, int WTM, int WTN,
+          int NBM, int NBN>
+__device__ __forceinline__ void store_tile(const GemmArgs<T>& p, typename MF::acc_t (&acc)[NBM][NBN],
+                                  const TileUnit& t, int m0, int n0, int wm0, int wn0, int lane,
+                                  T* C)
+{
+    // Whole tile: C = alpha*acc + beta*C (C is not read when beta == 0).
+    // Split unit: the raw fp partial goes to its BM x BN slot of the
+    // workspace (row-major, tile-local); splitk_reduce_kernel finishes C.
+    // With B n-contiguous, a lane owns UB consecutive columns of each row and
+    // writes them with one vector store when the destination allows it.
+    constexpr int UB = MapB::U, MB = MF::MB;
+    const int q = lane / MB, jl = lane % MB;
+    typedef typename Glob<T>::type GT;
+    GT* dst;
+    int64_t ldd;
+    int row_lim, col_lim;
+    T alpha, beta;
+    bool vec_ok;
+    bool relu = false;
+    // triangle window of a row: columns [m + lo_off, m + hi_off] of the tile
+    // stay (local column c of local row m is global column n0 + c, row m0 + m)
+    int lo_off = -(1 << 30), hi_off = 1 << 30;
+    if (t.is_split) {
+        // batch entry z's partials follow those of entries 0 .. z-1
+        const int64_t slot = (int64_t)blockIdx.z * (p.tiles - p.num_full) + (t.id - p.num_full);
+        dst = (GT*)(p.ws + (slot * p.split + t.part) * (BM * BN));
+        ldd = BN;
+        row_lim = BM;
+        col_lim = BN;
+        alpha = (T)1;
+        beta = (T)0;
+        vec_ok = true;
+    } else {
+        dst = (GT*)(C + (int64_t)m0 * p.ldc + n0);
+        ldd = p.ldc;
+        row_lim = p.M - m0;
+        col_lim = p.N - n0;
+        alpha = p.alpha;
+        beta = p.beta;
+        vec_ok = p.c_vec;
+        relu = p.relu != 0;
+        if (p.uplo == 1) hi_off = m0 - n0;       // column <= row
+        else if (p.uplo == 2) lo_off = m0 - n0;  // column >= row
+    }
+    const bool read_c = beta != (T)0;
+
+    // A wave tile wholly inside C (and inside the triangle window) -- every
+    // split unit and every tile of a large problem but the edges -- takes a
+    // path without per-element tests: a block row's C loads are all issued
+    // before the first of them is used.  Rows that allow vector access use
+    // UB-wide loads and stores, others UB single ones.  (Under the general
+    // path's per-element branches each load waited for its own round trip
+    // before the next was issued: ~18 us per round of 256x256 tiles at
+    // 8192^3 with beta != 0.)
+    const bool interior = wm0 + WTM <= row_lim && wn0 + WTN <= col_lim &&
+                          wn0 + WTN - 1 <= wm0 + hi_off && wn0 >= wm0 + WTM - 1 + lo_off;
+    if (interior) {
+        constexpr int NS = NBN / UB;
+        auto finish = [&](auto WITH_C, auto VEC) {
+            typedef typename std::conditional<decltype(VEC)::value, CVec<T, UB>, CElems<T, UB>>::type CV;
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                T cv[NS][MF::NACC][UB];
+                if constexpr (decltype(WITH_C)::value) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+#pragma unroll
+                        for (int r = 0; r < MF::NACC; ++r) {
+                            const int m = wm0 + MapA::map(i, MF::row(r, q));
+                            const int nb = wn0 + MapB::map(s * UB, jl);
+                            CV::load(dst + (int64_t)m * ldd + nb, cv[s][r]);
+                        }
+                }
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+#pragma unroll
+                    for (int r = 0; r < MF::NACC; ++r) {
+                        const int m = wm0 + MapA::map(i, MF::row(r, q));
+                        const int nb = wn0 + MapB::map(s * UB, jl);
+                        T v[UB];
+#pragma unroll
+                        for (int u = 0; u < UB; ++u) {
+                            v[u] = alpha * acc[i][s * UB + u][r];
+                            if constexpr (decltype(WITH_C)::value) v[u] += beta * cv[s][r][u];
+                            if (relu) v[u] = relu_of(v[u]);
+                        }
+                        CV::store(dst + (int64_t)m * ldd + nb, v);
+                    }
+            }
+        };
+        if (UB == 1 || vec_ok) {
+            if (read_c) finish(Int<1>{}, std::true_type{});
+            else finish(Int<0>{}, std::true_type{});
+        } else {
+            if (read_c) finish(Int<1>{}, std::false_type{});
+            else finish(Int<0>{}, std::false_type{});
+        }
+        return;
+    }
+
+#pragma unroll
+    for (int i = 0; i < NBM; ++i)
+#pragma unroll
+        for (int s = 0; s < NBN / UB; ++s) {
+            const int nb = wn0 + MapB::map(s * UB, jl);
+#pragma unroll
+            for (int r = 0; r < MF::NACC; ++r) {
+                const int m = wm0 + MapA::map(i, MF::row(r, q));
+                if (m >= row_lim) continue;
+                const int c_lo = max(0, m + lo_off);
+                const int c_hi = min(col_lim, m + hi_off + 1);
+                const bool vec = UB > 1 && vec_ok && nb >= c_lo && nb + UB <= c_hi;
+                GT* cp = dst + (int64_t)m * ldd + nb;
+                T v[UB];
+#pragma unroll
+                for (int u = 0; u < UB; ++u) v[u] = alpha * acc[i][s * UB + u][r];
+                if (vec) {
+                    if (read_c) {
+                        T c[UB];
+                        CVec<T, UB>::load(cp, c);
+#pragma unroll
+                        for (int u = 0; u < UB; ++u) v[u] += beta * c[u];
+                    }
+                    if (relu) {
+#pragma unroll
+                        for (int u = 0; u < UB; ++u) v[u] = relu_of(v[u]);
+                    }
+                    CVec<T, UB>::store(cp, v);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < UB; ++u)
+                        if (nb + u >= c_lo && nb + u < c_hi) {
+                            T w = v[u];
+                            if (read_c) w += beta * cp[u];
+                            cp[u] = relu ? relu_of(w) : w;
+                        }
+                }
+            }
+        }
+}
+
 // Slice x of n items cut into `slots` near-equal slices, in order.
 __host__ __device__ constexpr int slice(int x, int n, int slots)
 {
@@ -661,22 +836,8 @@ gemm_mfma_kernel(GemmArgs<T> p)
     const int wm0 = (wave / WAVES_N) * WTM;
     const int wn0 = (wave % WAVES_N) * WTN;
 
-    // ---- tile index: XCD-aware remap, then GROUP_M-tall column walk ----
-    // Blocks [0, num_full) own whole tiles; the rest are (tile, k-part) units.
-    int id = blockIdx.x;
-    int part = 0;
-    const bool is_split = id >= p.num_full;
-    if (is_split) {
-        const int u = id - p.num_full;
-        id = p.num_full + u / p.split;
-        part = u - (u / p.split) * p.split;
-    } else if ((p.num_full & 7) == 0) {
-        const int per_xcd = p.num_full >> 3;
-        id = (id & 7) * per_xcd + (id >> 3);
-    }
-    int tm, tn;
-    tile_coords(p, id, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN;
+    const TileUnit t = tile_unit(p);
+    const int m0 = t.tm * BM, n0 = t.tn * BN;
 
     const T* A;
     const T* B;
@@ -709,8 +870,8 @@ gemm_mfma_kernel(GemmArgs<T> p)
 
     // k tiles [kt0, nk) of this block (a k-part for split units)
     const int nk_all = (p.K + BK - 1) / BK;
-    const int kt0 = is_split ? (int)((int64_t)part * nk_all / p.split) : 0;
-    const int nk = is_split ? (int)((int64_t)(part + 1) * nk_all / p.split) : nk_all;
+    const int kt0 = t.is_split ? (int)((int64_t)t.part * nk_all / p.split) : 0;
+    const int nk = t.is_split ? (int)((int64_t)(t.part + 1) * nk_all / p.split) : nk_all;
 
     // Fixed descriptors at the tile's k = 0 origin, for the k tiles that are
     // full and not the last (see the main loop).  Usable when every offset
@@ -892,141 +1053,7 @@ gemm_mfma_kernel(GemmArgs<T> p)
 
     probe_mark(p, 1);  // end of the k loop
 
-    // ---- epilogue ----
-    // Whole tile: C = alpha*acc + beta*C (C is not read when beta == 0).
-    // Split unit: the raw fp partial goes to its BM x BN slot of the
-    // workspace (row-major, tile-local); splitk_reduce_kernel finishes C.
-    // With B n-contiguous, a lane owns UB consecutive columns of each row and
-    // writes them with one vector store when the destination allows it.
-    constexpr int UB = FragB::U;
-    const int q = lane / MB, jl = lane % MB;
-    typedef typename Glob<T>::type GT;
-    GT* dst;
-    int64_t ldd;
-    int row_lim, col_lim;
-    T alpha, beta;
-    bool vec_ok;
-    bool relu = false;
-    // triangle window of a row: columns [m + lo_off, m + hi_off] of the tile
-    // stay (local column c of local row m is global column n0 + c, row m0 + m)
-    int lo_off = -(1 << 30), hi_off = 1 << 30;
-    if (is_split) {
-        // batch entry z's partials follow those of entries 0 .. z-1
-        const int64_t slot = (int64_t)blockIdx.z * (p.tiles - p.num_full) + (id - p.num_full);
-        dst = (GT*)(p.ws + (slot * p.split + part) * (BM * BN));
-        ldd = BN;
-        row_lim = BM;
-        col_lim = BN;
-        alpha = (T)1;
-        beta = (T)0;
-        vec_ok = true;
-    } else {
-        dst = (GT*)(C + (int64_t)m0 * p.ldc + n0);
-        ldd = p.ldc;
-        row_lim = p.M - m0;
-        col_lim = p.N - n0;
-        alpha = p.alpha;
-        beta = p.beta;
-        vec_ok = p.c_vec;
-        relu = p.relu != 0;
-        if (p.uplo == 1) hi_off = m0 - n0;       // column <= row
-        else if (p.uplo == 2) lo_off = m0 - n0;  // column >= row
-    }
-    const bool read_c = beta != (T)0;
-
-    // A wave tile wholly inside C (and inside the triangle window) -- every
-    // split unit and every tile of a large problem but the edges -- takes a
-    // path without per-element tests: a block row's C loads are all issued
-    // before the first of them is used.  Rows that allow vector access use
-    // UB-wide loads and stores, others UB single ones.  (Under the general
-    // path's per-element branches each load waited for its own round trip
-    // before the next was issued: ~18 us per round of 256x256 tiles at
-    // 8192^3 with beta != 0.)
-    const bool interior = wm0 + WTM <= row_lim && wn0 + WTN <= col_lim &&
-                          wn0 + WTN - 1 <= wm0 + hi_off && wn0 >= wm0 + WTM - 1 + lo_off;
-    if (interior) {
-        constexpr int NS = NBN / UB;
-        auto finish = [&](auto WITH_C, auto VEC) {
-            typedef typename std::conditional<decltype(VEC)::value, CVec<T, UB>, CElems<T, UB>>::type CV;
-#pragma unroll
-            for (int i = 0; i < NBM; ++i) {
-                T cv[NS][MF::NACC][UB];
-                if constexpr (decltype(WITH_C)::value) {
-#pragma unroll
-                    for (int s = 0; s < NS; ++s)
-#pragma unroll
-                        for (int r = 0; r < MF::NACC; ++r) {
-                            const int m = wm0 + FragA::map(i, MF::row(r, q));
-                            const int nb = wn0 + FragB::map(s * UB, jl);
-                            CV::load(dst + (int64_t)m * ldd + nb, cv[s][r]);
-                        }
-                }
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-#pragma unroll
-                    for (int r = 0; r < MF::NACC; ++r) {
-                        const int m = wm0 + FragA::map(i, MF::row(r, q));
-                        const int nb = wn0 + FragB::map(s * UB, jl);
-                        T v[UB];
-#pragma unroll
-                        for (int u = 0; u < UB; ++u) {
-                            v[u] = alpha * acc[i][s * UB + u][r];
-                            if constexpr (decltype(WITH_C)::value) v[u] += beta * cv[s][r][u];
-                            if (relu) v[u] = relu_of(v[u]);
-                        }
-                        CV::store(dst + (int64_t)m * ldd + nb, v);
-                    }
-            }
-        };
-        if (UB == 1 || vec_ok) {
-            if (read_c) finish(Int<1>{}, std::true_type{});
-            else finish(Int<0>{}, std::true_type{});
-        } else {
-            if (read_c) finish(Int<1>{}, std::false_type{});
-            else finish(Int<0>{}, std::false_type{});
-        }
-        return;
-    }
-
-#pragma unroll
-    for (int i = 0; i < NBM; ++i)
-#pragma unroll
-        for (int s = 0; s < NBN / UB; ++s) {
-            const int nb = wn0 + FragB::map(s * UB, jl);
-#pragma unroll
-            for (int r = 0; r < MF::NACC; ++r) {
-                const int m = wm0 + FragA::map(i, MF::row(r, q));
-                if (m >= row_lim) continue;
-                const int c_lo = max(0, m + lo_off);
-                const int c_hi = min(col_lim, m + hi_off + 1);
-                const bool vec = UB > 1 && vec_ok && nb >= c_lo && nb + UB <= c_hi;
-                GT* cp = dst + (int64_t)m * ldd + nb;
-                T v[UB];
-#pragma unroll
-                for (int u = 0; u < UB; ++u) v[u] = alpha * acc[i][s * UB + u][r];
-                if (vec) {
-                    if (read_c) {
-                        T c[UB];
-                        CVec<T, UB>::load(cp, c);
-#pragma unroll
-                        for (int u = 0; u < UB; ++u) v[u] += beta * c[u];
-                    }
-                    if (relu) {
-#pragma unroll
-                        for (int u = 0; u < UB; ++u) v[u] = relu_of(v[u]);
-                    }
-                    CVec<T, UB>::store(cp, v);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < UB; ++u)
-                        if (nb + u >= c_lo && nb + u < c_hi) {
-                            T w = v[u];
-                            if (read_c) w += beta * cp[u];
-                            cp[u] = relu ? relu_of(w) : w;
-                        }
-                }
-            }
-        }
+    store_tile<T, MF, FragA, FragB, BM, BN, WTM, WTN, NBM, NBN>(p, acc, t, m0, n0, wm0, wn0, lane, C);
 }
 
 // Split-K finish: for tail tile `slot` (tile id num_full + slot), sum the

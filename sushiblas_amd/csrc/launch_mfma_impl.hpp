@@ -7,6 +7,21 @@
 
 namespace sbx {
 
+// The second kernel of a split call (none otherwise), and the launches' status.
+template <typename T, int BM, int BN>
+hipError_t launch_reduce(const GemmArgs<T>& a, int batch, hipStream_t stream)
+{
+    if (a.split > 1) {
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        // 256 threads per block whatever the tile's waves
+        constexpr int CHUNKS = SplitReduce<T, BM, BN>::CHUNKS;
+        const dim3 rgrid((unsigned)((a.tiles - a.num_full) * CHUNKS), 1, (unsigned)batch);
+        splitk_reduce_kernel<T, BM, BN><<<rgrid, dim3(256), 0, stream>>>(a);
+    }
+    return hipGetLastError();
+}
+
 template <typename T, int BM, int BN, int BK, int WM, int WN, int PF, int WPE, int MI, int BNC,
           int BMC>
 hipError_t launch_mfma(const GemmArgs<T>& a, bool a_kc, bool b_kc, int batch, hipStream_t stream)
@@ -44,15 +59,7 @@ hipError_t launch_mfma(const GemmArgs<T>& a, bool a_kc, bool b_kc, int batch, hi
         SBX_LAUNCH(false, false, false);
     }
 #undef SBX_LAUNCH
-    if (a.split > 1) {
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        // the reduction runs 256 threads per block whatever the tile's waves
-        constexpr int CHUNKS = SplitReduce<T, BM, BN>::CHUNKS;
-        const dim3 rgrid((unsigned)((tiles - a.num_full) * CHUNKS), 1, (unsigned)batch);
-        splitk_reduce_kernel<T, BM, BN><<<rgrid, dim3(256), 0, stream>>>(a);
-    }
-    return hipGetLastError();
+    return launch_reduce<T, BM, BN>(a, batch, stream);
 }
 
 }  // namespace sbx

@@ -611,30 +611,37 @@ struct WorkspaceLease {
     ~WorkspaceLease() { release(); }
 };
 
+// The fp32 tiles that are 48 wide and more both ways and 128 one way multiply
+// on the bf16 matrix cores (gemm_split.hpp): 1.1-1.6 times as fast as on the
+// fp32 ones from K = 128 on (8192^3 7.14 -> 4.64 ms; 2048^2 x 128 14.7 -> 12.5
+// us, 65536 x 64 x 512 37.3 -> 31).  The 32-wide tiles, bound by HBM, and the
+// 64-wide ones of 64 and 128 stay on fp32 MFMAs: with one short workgroup per
+// CU the split's longer way from memory to an MFMA has nothing beside it
+// (1024^3 on 64^2 tiles 19.4 us against 21.8, 33870 x 9 x 1420 51.7 against 55.2).
 hipError_t launch_cfg(Cfg cfg, GemmArgs<float>& a, bool akc, bool bkc, const Problem& p,
                       int nb, hipStream_t s)
 {
     switch (cfg) {
     case F32_256x256:
-        return launch_mfma<float, 256, 256, 32, 4, 2, 1, 2>(a, akc, bkc, nb, s);
+        return launch_split<256, 256, 8, 1, 1, 2>(a, akc, bkc, nb, s);
     case F32_256x128:
-        return launch_mfma<float, 256, 128, 16, 4, 1, 2, 2>(a, akc, bkc, nb, s);
+        return launch_split<256, 128, 4, 1, 1, 2>(a, akc, bkc, nb, s);
     case F32_128x128:
-        return launch_mfma<float, 128, 128, 16, 2, 2, 2, 2>(a, akc, bkc, nb, s);
+        return launch_split<128, 128, 4, 1, 2, 2>(a, akc, bkc, nb, s);
     case F32_128x128_O3:
-        return launch_mfma<float, 128, 128, 16, 2, 2, 2, 3>(a, akc, bkc, nb, s);
+        return launch_split<128, 128, 4, 1, 1, 3>(a, akc, bkc, nb, s);
     case F32_128x64:
         return launch_mfma<float, 128, 64, 32, 2, 2, 2, 2>(a, akc, bkc, nb, s);
     case F32_256x64:
-        return launch_mfma<float, 256, 64, 32, 8, 1, 2, 2, 1>(a, akc, bkc, nb, s);
+        return launch_split<256, 64, 8, 1, 2, 2>(a, akc, bkc, nb, s);
     case F32_256x48:
-        return launch_mfma<float, 256, 64, 32, 8, 1, 2, 2, 1, 48>(a, akc, bkc, nb, s);
+        return launch_split<256, 64, 8, 1, 2, 2, 48>(a, akc, bkc, nb, s);
     case F32_64x128:
         return launch_mfma<float, 64, 128, 32, 2, 2, 2, 2>(a, akc, bkc, nb, s);
     case F32_64x256:
-        return launch_mfma<float, 64, 256, 32, 1, 8, 2, 2, 1>(a, akc, bkc, nb, s);
+        return launch_split<64, 256, 1, 8, 2, 2>(a, akc, bkc, nb, s);
     case F32_48x256:
-        return launch_mfma<float, 64, 256, 32, 1, 8, 2, 2, 1, 256, 48>(a, akc, bkc, nb, s);
+        return launch_split<64, 256, 1, 8, 2, 2, 256, 48>(a, akc, bkc, nb, s);
     case F32_128x32:
         return launch_mfma<float, 128, 32, 32, 4, 1, 2, 2, 1>(a, akc, bkc, nb, s);
     case F32_32x128:

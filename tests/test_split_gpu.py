@@ -1,0 +1,112 @@
+"""GPU checks of the fp32 tiles that multiply on the bf16 matrix cores
+(gemm_split.hpp): each tile by name at sizes around its edges, K tails and
+every transpose against the oracle accumulating in double; an error no larger
+than fp32 sums in order leave; and the operands the split cannot hold
+(infinities, NaN, values past bf16's largest, rows and columns below 2^-100),
+which the kernel computes again with fp32 MFMAs."""
+import numpy as np
+import pytest
+
+import oracle
+from gemm_cases import TOL, c_window, make_inputs, normwise, run_oracle, run_sbx
+
+pytestmark = pytest.mark.gpu
+
+SEED = 20261240
+
+# plan, m, n, k: one tile short, one past, ragged; K from a part of a k tile on
+TILES = [
+    ("mfma_f32_256x128x16_w4x1", 255, 129, 96), ("mfma_f32_256x128x16_w4x1", 513, 260, 1031),
+    ("mfma_f32_256x128x16_w4x1", 300, 140, 31), ("mfma_f32_256x128x16_w4x1+splitk3", 130, 127, 333),
+    ("mfma_f32_128x128x16_w2x2", 127, 129, 33), ("mfma_f32_128x128x16_w2x2", 257, 130, 1030),
+    ("mfma_f32_128x128x16_w2x2+splitk2", 100, 131, 64), ("mfma_f32_128x128x16_w2x2_o3", 129, 255, 65),
+    ("mfma_f32_128x128x16_w2x2_o3", 1, 2, 700), ("mfma_f32_128x128x16_w2x2_o3+splitk5", 260, 3, 403),
+    ("mfma_f32_256x64x32_w8x1", 257, 63, 127), ("mfma_f32_256x64x32_w8x1+splitk2", 300, 5, 1025),
+    ("mfma_f32_256x48x32_w8x1", 511, 47, 129), ("mfma_f32_64x256x32_w1x8", 61, 257, 98),
+    ("mfma_f32_48x256x32_w1x8+splitk2", 40, 257, 1026), ("mfma_f32_256x256x32_w4x2", 257, 255, 163),
+]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_split_tiles_match_the_oracle(cuda, ta, tb):
+    for i, (plan, m, n, k) in enumerate(TILES):
+        off = ((0, 0, 0), (1, 2, 3))[i % 2]
+        A, lda, B, ldb, C, ldc = make_inputs(np.float32, 0, ta, tb, m, n, k, SEED + i, pad=(3, 5, 2))
+        C0 = C.copy()
+        print(f"split case {m}x{n}x{k} t{ta}{tb} -> {plan}", flush=True)
+        got = run_sbx(cuda, np.float32, 0, ta, tb, m, n, k, 1.25, A, lda, B, ldb, -0.5, C, ldc,
+                      offsets=off, plan=plan)
+        want = run_oracle(0, ta, tb, m, n, k, 1.25, A, lda, B, ldb, -0.5, C0, ldc)
+        assert normwise(0, got, want, m, n, ldc) <= TOL[np.float32], plan
+        pad = np.ones(C.size, bool)
+        for r in range(m):
+            pad[r * ldc:r * ldc + n] = False
+        np.testing.assert_array_equal(got[pad], C0[pad])
+
+
+@pytest.mark.parametrize("dist", ["uniform", "normal", "positive"])
+def test_split_error_is_below_fp32_sums(cuda, dist):
+    """Against double sums, the tile is no further off than the fp32 kernel
+    that sums in order (the generic one), 64 to 4096 terms."""
+    for i, k in enumerate((64, 257, 1000, 4096)):
+        m, n = 256, 128
+        A, lda, B, ldb, C, ldc = make_inputs(np.float32, 0, 0, 0, m, n, k, SEED + 40 + i,
+                                             dist="normal" if dist == "normal" else "uniform")
+        if dist == "positive":
+            A, B = np.abs(A), np.abs(B)
+        want = A.reshape(m, lda)[:, :k].astype(np.float64) @ B.reshape(k, ldb)[:, :n].astype(np.float64)
+        errs = []
+        for kw in ({"plan": "mfma_f32_256x128x16_w4x1"}, {"algo": 1}):
+            got = run_sbx(cuda, np.float32, 0, 0, 0, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, **kw)
+            d = got.reshape(m, ldc)[:, :n].astype(np.float64) - want
+            errs.append(float(np.linalg.norm(d) / np.linalg.norm(want)))
+        print(f"{dist} k={k}: split {errs[0]:.2e}, fp32 in order {errs[1]:.2e}", flush=True)
+        assert errs[0] <= errs[1]
+
+
+PLANS = ["mfma_f32_256x128x16_w4x1", "mfma_f32_128x128x16_w2x2", "mfma_f32_128x128x16_w2x2_o3+splitk2",
+         "mfma_f32_256x64x32_w8x1", "mfma_f32_64x256x32_w1x8"]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("plan", PLANS)
+def test_operands_the_split_cannot_hold(cuda, plan, ta, tb):
+    m, n, k = 270, 150, 200
+    A, lda, B, ldb, C, ldc = make_inputs(np.float32, 0, ta, tb, m, n, k, SEED + 60)
+    opa = A.reshape(k, lda).T if ta else A.reshape(m, lda)   # views: writes go to A, B
+    opb = B.reshape(n, ldb).T if tb else B.reshape(k, ldb)
+    opa[3, 17] = np.inf
+    opa[5, 199] = np.nan
+    opb[100, 70] = -np.inf
+    opa[9, :] = np.float32(3.4e38)       # rounds to an infinite bf16
+    opb[:, 7] *= np.float32(1e-6)
+    opa[20, :] *= np.float32(1e-36)      # a row below 2^-100: pieces would lose bits
+    opa[21, :] = 0.0
+    opb[:, 9] *= np.float32(1e-34)
+    opa[30, 40] = np.float32(1e-36)      # one tiny value in an ordinary row
+    got = run_sbx(cuda, np.float32, 0, ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, plan=plan)
+    got = c_window(0, got, m, n, ldc).astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = opa.astype(np.float64) @ opb.astype(np.float64)
+    # every sum past fp32's largest is far past it or far below it here,
+    # except row 9's: k values of 3.4e38 times [-1, 1)
+    free = np.zeros((m, n), bool)
+    free[9, :] = True
+    free[9, 7] = free[9, 9] = False      # ... which these two columns scale back into range
+    nan = np.isnan(want)
+    inf = np.isinf(want)
+    np.testing.assert_array_equal(np.isnan(got) & ~free, nan & ~free)
+    np.testing.assert_array_equal(got[inf & ~free], want[inf & ~free])
+    fin = np.isfinite(want) & ~free
+    assert np.isfinite(got[fin]).all()
+    for r in range(m):  # row by row, so that the tiny row counts by itself
+        for cols in ([9], [c for c in range(n) if c != 9]):
+            f = [c for c in cols if fin[r, c]]
+            if not f:
+                continue
+            scale = np.abs(opa[r].astype(np.float64)) @ np.abs(opb[:, f].astype(np.float64))
+            with np.errstate(invalid="ignore"):
+                e = np.abs(got[r, f] - want[r, f])
+            # |error| <= 1e-6 of the sum of magnitudes (200 terms); results below
+            # 2^-126 are rounded to multiples of 2^-149
+            assert (e <= 1e-6 * scale + 2.0 ** -149 * k).all(), (r, float((e / (scale + 1e-300)).max()))
