@@ -55,17 +55,21 @@ struct Problem {
     int table_swap;
 };
 
-// Tile configurations compiled into the library (gemm_cfg_*.hip).
+// Tile configurations compiled into the library (gemm_cfg_*.hip).  The names
+// (kCfg) are the plans' handles in sbx_gemm_ex_plan and keep the tile, k step
+// and wave grid of the fp32 MFMA kernel they began with; the fp32 tiles that
+// multiply on the bf16 matrix cores (see launch_cfg) have the tile the name
+// says, a k step of 32 and one wave along one dimension.
 enum Cfg {
-    F32_256x256,   // large fp32: 8 waves of 64x128, 2 waves/SIMD (128 accumulators)
-    F32_256x128,   // large fp32: 4 waves of 64x128, two workgroups per CU, 2 tiles in flight
-    F32_128x128,   // mid-size fp32: 4 waves of 64x64, 2 waves/SIMD, 2 tiles in flight
+    F32_256x256,   // fp32 SYRK, and pairs of 256x128: 8 waves of 32x256 (128 accumulators)
+    F32_256x128,   // large fp32: 4 waves of 64x128, two workgroups per CU
+    F32_128x128,   // mid-size fp32: 4 waves of 32x128, 2 waves/SIMD, 2 tiles in flight
     F32_128x128_O3,  // the same tile at 3 waves/SIMD (three workgroups per CU)
     F32_128x64,    // n <= 64 (tall-skinny): 4 waves of 64x32, 2 tiles in flight
-    F32_256x64,    // n <= 64 with a full round of 256-row tiles: 8 waves of 32x64 (16x16x4 MFMAs)
+    F32_256x64,    // n <= 64 with a full round of 256-row tiles: 8 waves of 32x64
     F32_256x48,    // 32 < n <= 48: the 256x64 tile computing 48 columns (waves of 32x48)
     F32_64x128,    // m <= 64
-    F32_64x256,    // m <= 64 with a full round of 256-column tiles: 8 waves of 64x32 (16x16x4 MFMAs)
+    F32_64x256,    // m <= 64 with a full round of 256-column tiles: 8 waves of 64x32
     F32_48x256,    // 32 < m <= 48: the 64x256 tile computing 48 rows (waves of 48x32)
     F32_128x32,    // n <= 32: 4 waves of 32x32 (16x16x4 MFMAs)
     F32_32x128,    // m <= 32: 4 waves of 32x32 (16x16x4 MFMAs)
@@ -229,8 +233,10 @@ bool mfma_feasible(const Problem& p, Cfg c)
     if (c == F32_256x48 && p.n > 48) return false;
     if (c == F32_48x256 && p.m > 48) return false;  // and of rows
     const size_t elem = p.dtype == SBX_F32 ? 4 : 8;
-    return offsets_fit(!p.ta, ci.bm, ci.bk, p.lda, elem) &&
-           offsets_fit(p.tb, ci.bn, ci.bk, p.ldb, elem) &&
+    // (the fp32 tiles whose name says 16 walk 32 k at a time on the bf16 cores)
+    const int bk = p.dtype == SBX_F32 ? 32 : ci.bk;
+    return offsets_fit(!p.ta, ci.bm, bk, p.lda, elem) &&
+           offsets_fit(p.tb, ci.bn, bk, p.ldb, elem) &&
            cdiv(p.m, ci.bm) * cdiv(p.n, ci.bn) < ((int64_t)1 << 31);
 }
 
@@ -618,6 +624,28 @@ struct WorkspaceLease {
 // 64-wide ones of 64 and 128 stay on fp32 MFMAs: with one short workgroup per
 // CU the split's longer way from memory to an MFMA has nothing beside it
 // (1024^3 on 64^2 tiles 19.4 us against 21.8, 33870 x 9 x 1420 51.7 against 55.2).
+// Whether an unsplit 256x128 plan, two tiles per CU, runs its tiles in
+// neighbouring pairs, one 8-wave workgroup of 256x256 per CU.  The pair shares
+// each split of B among twice the rows and each wave's split of A among twice
+// the columns: 23 % fewer vector instructions per MFMA, and as the chip's
+// power bounds both, 8192^3 runs 4.37 against 4.69 ms, 4096^3 556 against 591
+// us, 4096^2 x 1024 149.5 against 153.5.  From K = 1024 on (8192^2 x 256 181 against
+// 177 us: one workgroup has no other to overlap its prologue and epilogue
+// with), and where the pairs make no more rounds than the tiles (9000^2 x
+// 3000, 6 rounds against 5: 2378 against 2238 us).
+constexpr int kPairMinK = 1024;
+
+bool tiles_in_pairs(const GemmArgs<float>& a, int nb)
+{
+    if (a.split != 1 || a.uplo || a.K < kPairMinK) return false;
+    const int64_t cus = cu_count();
+    const int64_t pairs = (int64_t)a.tiles_m * ((a.tiles_n + 1) / 2) * nb;
+    return cdiv(pairs, cus) <= cdiv((int64_t)a.tiles * nb, 2 * cus) &&
+           // the pair's offsets into a k-major B span 256 columns, into a
+           // k-contiguous one 256 rows
+           offsets_fit(true, 256, 32, a.ldb, 4);
+}
+
 hipError_t launch_cfg(Cfg cfg, GemmArgs<float>& a, bool akc, bool bkc, const Problem& p,
                       int nb, hipStream_t s)
 {
@@ -625,6 +653,12 @@ hipError_t launch_cfg(Cfg cfg, GemmArgs<float>& a, bool akc, bool bkc, const Pro
     case F32_256x256:
         return launch_split<256, 256, 8, 1, 1, 2>(a, akc, bkc, nb, s);
     case F32_256x128:
+        if (tiles_in_pairs(a, nb)) {
+            a.tiles_n = (a.tiles_n + 1) / 2;
+            a.tiles = a.num_full = a.tiles_m * a.tiles_n;
+            a.group_m = a.tiles_m < 8 ? a.tiles_m : 8;
+            return launch_split<256, 256, 8, 1, 1, 2>(a, akc, bkc, nb, s);
+        }
         return launch_split<256, 128, 4, 1, 1, 2>(a, akc, bkc, nb, s);
     case F32_128x128:
         return launch_split<128, 128, 4, 1, 2, 2>(a, akc, bkc, nb, s);
