@@ -30,6 +30,12 @@
  *     propagate).
  *   - layout 0 = row-major, 1 = column-major (Core::Layout,
  *     include/SushiBLAS/core/common.hpp:41-45).  transA/transB: 0 or 1.
+ *   - fp32 GEMM and SYRK on tiles of 128 rows or columns and more multiply on
+ *     the bf16 matrix cores, each operand value as the exact sum of three
+ *     bf16 values: results are nearer to the exact sums than fp32 products
+ *     added in order (3.0e-7 against 1.6e-6 at K = 8192).  Infinities, NaN
+ *     and values near fp32's largest give what fp32 arithmetic gives; rows of
+ *     op(A) and columns of op(B) below 2^-100 as a whole keep full precision.
  *   - Re-entrant: the only global state is the per-device CU count and the
  *     workspace cache, both behind mutexes; safe to call from any host thread
  *     (the reference runs the GEMM closure on a scheduler worker thread).
@@ -205,8 +211,10 @@ int sbx_dsyrk_strided_batched(void* stream, int layout, int upper, int trans, in
                               int64_t str_a, double beta, double* C, int64_t ldc, int64_t str_c,
                               int64_t batch);
 
-/* Name of the kernel the dispatcher would launch for this problem (tiling
- * heuristics introspection for benchmarks).  Pointers are assumed 16-byte
+/* Name of the plan (kernel tile and k-split) the dispatcher would launch for
+ * this problem (tiling heuristics introspection for benchmarks).  A name is a
+ * plan's handle, not a description of the kernel's inside: an unsplit
+ * 256x128 plan may run its tiles in neighbouring pairs.  Pointers are assumed 16-byte
  * aligned.  Writes a NUL-terminated string of at most cap bytes. */
 int sbx_gemm_select(int dtype, int layout, int transA, int transB, int64_t m, int64_t n,
                     int64_t k, int64_t lda, int64_t ldb, int64_t ldc, char* name, size_t cap);

@@ -541,8 +541,9 @@ __device__ __forceinline__ bool split_failed(const GemmArgs<float>& p, typename 
 }
 
 // BM x BN tile, 32 k per step, WAVES_M x WAVES_N waves, one of them 1; BMC, BNC:
-// rows and columns of the tile that are computed (see gemm_mfma_kernel); PF:
-// see step1 and step; WPE: waves per SIMD; STREAM: the operand whose loads
+// rows and columns of the tile that are computed (fewer than BM, BN where the
+// host knows that M <= BMC or N <= BNC, one tile row or column: a 48-wide C
+// then does not pay for 64 columns of MFMAs); PF: see step1 and step; WPE: waves per SIMD; STREAM: the operand whose loads
 // are non-temporal.
 // One wave along N: each wave's rows of A are its own (A_DIRECT; one along M:
 // its columns of B), and that operand goes from memory to the wave's

@@ -12,8 +12,7 @@
 
 namespace sbx {
 
-template <typename T, int BM, int BN, int BK, int WM, int WN, int PF, int WPE, int MI = 0,
-          int BNC = BN, int BMC = BM>
+template <typename T, int BM, int BN, int BK, int WM, int WN, int PF, int WPE, int MI = 0>
 hipError_t launch_mfma(const GemmArgs<T>& a, bool a_kc, bool b_kc, int batch, hipStream_t stream);
 
 // The same for the fp32 tiles on the bf16 matrix cores (gemm_split.hpp).

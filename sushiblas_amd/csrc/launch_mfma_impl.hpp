@@ -22,8 +22,7 @@ hipError_t launch_reduce(const GemmArgs<T>& a, int batch, hipStream_t stream)
     return hipGetLastError();
 }
 
-template <typename T, int BM, int BN, int BK, int WM, int WN, int PF, int WPE, int MI, int BNC,
-          int BMC>
+template <typename T, int BM, int BN, int BK, int WM, int WN, int PF, int WPE, int MI>
 hipError_t launch_mfma(const GemmArgs<T>& a, bool a_kc, bool b_kc, int batch, hipStream_t stream)
 {
     const int tiles = a.tiles;
@@ -40,10 +39,10 @@ hipError_t launch_mfma(const GemmArgs<T>& a, bool a_kc, bool b_kc, int batch, hi
 #define SBX_LAUNCH(AK, BKC, TAIL)                                                                 \
     do {                                                                                          \
         if (streamed)                                                                             \
-            gemm_mfma_kernel<T, BM, BN, BK, WM, WN, AK, BKC, TAIL, PF, WPE, MI, kStream, BNC, BMC>\
+            gemm_mfma_kernel<T, BM, BN, BK, WM, WN, AK, BKC, TAIL, PF, WPE, MI, kStream>          \
                 <<<grid, block, 0, stream>>>(a);                                                  \
         else                                                                                      \
-            gemm_mfma_kernel<T, BM, BN, BK, WM, WN, AK, BKC, TAIL, PF, WPE, MI, 0, BNC, BMC>      \
+            gemm_mfma_kernel<T, BM, BN, BK, WM, WN, AK, BKC, TAIL, PF, WPE, MI, 0>                \
                 <<<grid, block, 0, stream>>>(a);                                                  \
     } while (0)
     if (a_kc && b_kc) {
