@@ -30,12 +30,14 @@
  *     propagate).
  *   - layout 0 = row-major, 1 = column-major (Core::Layout,
  *     include/SushiBLAS/core/common.hpp:41-45).  transA/transB: 0 or 1.
- *   - fp32 GEMM and SYRK on tiles of 128 rows or columns and more multiply on
- *     the bf16 matrix cores, each operand value as the exact sum of three
- *     bf16 values: results are nearer to the exact sums than fp32 products
- *     added in order (3.0e-7 against 1.6e-6 at K = 8192).  Infinities, NaN
- *     and values near fp32's largest give what fp32 arithmetic gives; rows of
- *     op(A) and columns of op(B) below 2^-100 as a whole keep full precision.
+ *   - fp32 GEMM and SYRK on the tiles of 128x128, 256x64, 64x256 and more
+ *     multiply on the bf16 matrix cores, each operand value as the exact sum of
+ *     three bf16 values: results are nearer to the exact sums than fp32 products
+ *     added in order (3.0e-7 against 1.6e-6 at K = 8192).  Where the sum is not
+ *     exact (bits below 2^-133, which only values below 2^-110 have) and that
+ *     could move a result by 2^-24 of its terms' magnitudes, and where
+ *     infinities, NaN or values next to fp32's largest meet, the tile is
+ *     computed again with fp32 products: it then gives what fp32 arithmetic gives.
  *   - Re-entrant: the only global state is the per-device CU count and the
  *     workspace cache, both behind mutexes; safe to call from any host thread
  *     (the reference runs the GEMM closure on a scheduler worker thread).

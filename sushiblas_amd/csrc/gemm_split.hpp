@@ -1,12 +1,13 @@
 // gemm_split.hpp -- the fp32 tile GEMM kernel of gfx950, on its bf16 matrix
 // cores.
 //
-// An fp32 value x is the exact sum of three bf16 values (8 significant bits
-// each, rounded to nearest): x = x0 + x1 + x2 with |x1| <= 2^-9 |x0| and
-// |x2| <= 2^-18 |x0|.  A product of two such sums has nine terms; the six
-// with a weight of 2^-18 and above,
+// An fp32 value x of 2^-110 and above is the exact sum of three bf16 values (8
+// significant bits each, rounded to nearest): x = x0 + x1 + x2 with
+// |x1| <= 2^-8 |x0| and |x2| <= 2^-17 |x0|.  (Below that it is one if its last
+// bit is 2^-133 or more, bf16's smallest value; see redo_needed for the
+// others.)  A product of two such sums has nine terms; the six largest,
 //     a2 b0 + a0 b2 + a1 b1 + a1 b0 + a0 b1 + a0 b0,
-// leave out less than 2^-25 of |a b|.  Each is one bf16 MFMA; the six of a 32-k
+// leave out less than 2^-24 of |a b|.  Each is one bf16 MFMA; the six of a 32-k
 // tile add up from zero (the smallest terms among the first), and that sum
 // goes to the accumulator with one fp32 addition.  (Six MFMAs straight into
 // the accumulator are 5 % faster, and as exact as the fp32 MFMA chain for
@@ -46,8 +47,16 @@ __device__ inline f32x4 split_mma(bf16x8 a, bf16x8 b, f32x4 c)
 
 // Two fp32 values -> their three bf16 pieces, packed (first value in the low
 // half).  The differences are exact.  An infinity, or a value that rounds to
-// one, leaves NaNs; see gemm_split_kernel's checks.
-__device__ inline void split_pair(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2)
+// one, leaves NaNs (see redo_needed).
+// lost: gathers the last remainders' bits.  A remainder of 2^-126 and more has 8
+// significant bits and none in its word's lower half; a smaller one is a
+// multiple of 2^-149 whose bits below 2^-133, those that bf16 has no place for,
+// are that lower half.  So the split of every value was exact if and only if
+// the lower half of `lost` is still 0 (checked on the device over all
+// magnitudes from 2^-149 to 2^-90).
+template <bool IN_PLACE>
+__device__ inline void split_pair(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2,
+                                  uint32_t& lost)
 {
     auto pack = [](float x, float y) {
         const bf16x2 v = {(__bf16)x, (__bf16)y};
@@ -62,7 +71,27 @@ __device__ inline void split_pair(float a, float b, uint32_t& p0, uint32_t& p1, 
     p0 = pack(a, b);
     const float a1 = a - lo(p0), b1 = b - hi(p0);
     p1 = pack(a1, b1);
-    p2 = pack(a1 - lo(p1), b1 - hi(p1));
+    const float a2 = a1 - lo(p1), b2 = b1 - hi(p1);
+    // IN_PLACE: one instruction, where it stands.  As an expression the compiler
+    // keeps a whole tile's remainders to join them at its end: for both
+    // operands that spills, for the direct one alone it is the better schedule
+    // (64 x 65536 x 2048: 114 us in place).
+    if constexpr (IN_PLACE)
+        asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(a2), "v"(b2));
+    else
+        lost |= __builtin_bit_cast(uint32_t, a2) | __builtin_bit_cast(uint32_t, b2);
+    p2 = pack(a2, b2);
+}
+
+constexpr uint32_t kLostBits = 0xffff;
+
+// Largest magnitude among four values, and whether the split of one is inexact.
+__device__ inline void gather_stats(f32x4 w, float& mx, uint32_t& lost)
+{
+    mx = fmaxf(fmaxf(mx, fmaxf(fabsf(w[0]), fabsf(w[1]))), fmaxf(fabsf(w[2]), fabsf(w[3])));
+    uint32_t p0, p1, p2;
+    split_pair<true>(w[0], w[1], p0, p1, p2, lost);
+    split_pair<true>(w[2], w[3], p0, p1, p2, lost);
 }
 
 // The lane's index, computed anew at each use: what the k loop's tail and the
@@ -119,7 +148,7 @@ struct SplitOperand {
     static constexpr int BLK = 1024 + PAD;  // bytes of a block
     static constexpr int PLANE = (X / 16) * BLK;
     static constexpr int BYTES = 3 * PLANE;  // one k tile
-    static constexpr int NMAX = KC ? NG : XV;
+    static constexpr int NROW = KC ? NG : XV;  // rows a thread holds values of
     static_assert(NF % 4 == 0 && NF >= 4, "at least one group of 4 k per thread");
     static_assert(KC ? (RSTEP * NG == X && (NL == 1 || NL * RSTEP == 16 * U || NL == NG))
                      : (XCH % 8 == 0 && XCH * OSTEP * 2 == NTHR && OSTEP * NG == 4),
@@ -128,7 +157,7 @@ struct SplitOperand {
     int voff;       // byte offset from the tile's base; out of range where X is masked
     int row_bytes;  // KC: bytes between sweeps; !KC: between k rows
     int lds0[NL];           // LDS offsets of this thread's first NL groups
-    float mx[NMAX];         // largest magnitude seen per row (see split_failed)
+    uint32_t lost = 0;      // see split_pair
     typedef float xvec __attribute__((ext_vector_type(XV)));
     f32x4 stage[KC ? PF : 1][KC ? NG : 1];       // KC: PF tiles in flight, 4 k of a row each
     xvec xstage[KC ? 1 : PF][KC ? 1 : NG][4];  // !KC: likewise, XV rows at one k each
@@ -164,8 +193,6 @@ struct SplitOperand {
             const int slot = xl % (16 * U) / U ^ (KC ? 2 * o : 0);
             lds0[l] = blk * BLK + (o * 16 + slot) * 16 + h * 8;
         }
-#pragma unroll
-        for (int i = 0; i < NMAX; ++i) mx[i] = 0.0f;
     }
 
     // Load a k tile through `rs`, moved by the scalar byte offset `soff`.
@@ -200,39 +227,55 @@ struct SplitOperand {
         }
     }
 
-    // Split group g of staging set S and write its pieces to the k tile at `lds`.
-    // MASK: it may straddle K (a k-contiguous vector past K holds the next
+    // Four consecutive k of a row: group g of staging set S, its row u.
+    // MASK: they may straddle K (a k-contiguous vector past K holds the next
     // row's first elements).
+    template <int S, bool MASK>
+    __device__ inline f32x4 value(int g, int u, int k_rem) const
+    {
+        f32x4 w;
+        if constexpr (KC) {
+            w = stage[S][g];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = xstage[S][g][e][u];
+        }
+        if constexpr (KC && KTAIL && MASK) {
+            const int lim = k_rem - first_k();
+#pragma unroll
+            for (int d = 1; d < 4; ++d) w[d] = d < lim ? w[d] : 0.0f;
+        }
+        return w;
+    }
+
+    // Split group g of staging set S and write its pieces to the k tile at `lds`.
     template <int S, bool MASK>
     __device__ inline void store(char* lds, int g, int k_rem)
     {
 #pragma unroll
         for (int u = 0; u < XV; ++u) {
-            f32x4 w;
-            if constexpr (KC) {
-                w = stage[S][g];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = xstage[S][g][e][u];
-            }
-            if constexpr (KC && KTAIL && MASK) {
-                const int lim = k_rem - first_k();
-#pragma unroll
-                for (int d = 1; d < 4; ++d) w[d] = d < lim ? w[d] : 0.0f;
-            }
-            float& m = mx[KC ? g : u];
-            m = fmaxf(fmaxf(m, fabsf(w[0])), fabsf(w[1]));
-            m = fmaxf(fmaxf(m, fabsf(w[2])), fabsf(w[3]));
+            const f32x4 w = value<S, MASK>(g, u, k_rem);
             u32x2 p[3];
             uint32_t a0, a1, a2, b0, b1, b2;
-            split_pair(w[0], w[1], a0, a1, a2);
-            split_pair(w[2], w[3], b0, b1, b2);
+            split_pair<true>(w[0], w[1], a0, a1, a2, lost);
+            split_pair<true>(w[2], w[3], b0, b1, b2, lost);
             p[0] = u32x2{a0, b0}; p[1] = u32x2{a1, b1}; p[2] = u32x2{a2, b2};
             const int at = KC ? lds0[g % NL] + g / NL * (NL * RSTEP / 16) * BLK
                               : lds0[0] + u * BLK + g * OSTEP * 256;
 #pragma unroll
             for (int t = 0; t < 3; ++t) *reinterpret_cast<u32x2*>(lds + at + t * PLANE) = p[t];
         }
+    }
+
+    // The staged tile's part in its rows' statistics.
+    template <int S>
+    __device__ inline void stats(float (&mx)[NROW], uint32_t (&ls)[NROW], int k_rem)
+    {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int u = 0; u < XV; ++u)
+                gather_stats(value<S, true>(g, u, k_rem), mx[KC ? g : u], ls[KC ? g : u]);
     }
 
     // Tile row of slot i of block b.
@@ -246,8 +289,8 @@ struct SplitOperand {
         const int i = lane % 16, o = lane / 16;
         return (o * 16 + (KC ? i ^ (2 * o) : i)) * 16;
     }
-    // tile row of this thread's mx[i]
-    __device__ static inline int max_row(int tid, int i, int)
+    // tile row of this thread's row i
+    __device__ static inline int row_of(int tid, int i, int)
     {
         return KC ? tid / VPR + i * RSTEP : chunk(tid) * XV + i;
     }
@@ -273,9 +316,9 @@ struct DirectOperand {
     static constexpr int NPC = PF > 1 ? 2 : 1;
     static constexpr int U = NB % 4 == 0 ? 4 : NB % 2 == 0 ? 2 : 1;
     static constexpr int NW = KC ? 1 : NB / U;  // !KC: groups of interleaved blocks
-    static constexpr int NMAX = NB;
+    static constexpr int NROW = NB;  // rows a lane holds values of
     int voff[KC ? 2 : NW];
-    float mx[NB];
+    uint32_t lost = 0;  // see split_pair
     typedef float xvec __attribute__((ext_vector_type(U)));
     f32x4 stage[KC ? PF : 1][KC ? NB : 1][2];     // KC: PF tiles in flight
     xvec xstage[KC ? 1 : PF][KC ? 1 : NW][8];  // !KC: likewise, U rows at one k each
@@ -301,8 +344,6 @@ struct DirectOperand {
                 voff[w] = x < x_rem ? (int)((k0 * ld + x) * 4) : kOobOffset;
             }
         }
-#pragma unroll
-        for (int b = 0; b < NB; ++b) mx[b] = 0.0f;
     }
 
     // A k tile through rs[b] (KC: block b's descriptor; else rs[0]).
@@ -345,9 +386,9 @@ struct DirectOperand {
         }
     }
 
-    // Split the staged tile into the MFMA operands pc[P].
-    template <int S, int P, bool MASK>
-    __device__ inline void split(int k_rem)
+    // The trade of halves, once per staged tile, before value().
+    template <int S>
+    __device__ inline void arrange()
     {
         if constexpr (TRADE)
 #pragma unroll
@@ -363,26 +404,39 @@ struct DirectOperand {
                     stage[S][b][1][d] = __builtin_bit_cast(
                         float, __builtin_amdgcn_update_dpp(y, x, kRor8, 0xf, 0x3, false));
                 }
+    }
+
+    // k = 16h + 4q + 0..3 of block b's row.  MASK: they may straddle K.
+    template <int S, bool MASK>
+    __device__ inline f32x4 value(int b, int h, int k_rem) const
+    {
+        f32x4 w;
+        if constexpr (KC) {
+            w = stage[S][b][h];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = xstage[S][b / U][4 * h + e][b % U];
+        }
+        if constexpr (KC && KTAIL && MASK) {
+            const int lim = k_rem - first_k() - 16 * h;
+#pragma unroll
+            for (int d = 1; d < 4; ++d) w[d] = d < lim ? w[d] : 0.0f;
+        }
+        return w;
+    }
+
+    // Split the staged tile into the MFMA operands pc[P].
+    template <int S, int P, bool MASK>
+    __device__ inline void split(int k_rem)
+    {
+        arrange<S>();
         u32x4 p[NB][3];
         auto half = [&](int b, int h) SBX_INLINE {
-            f32x4 w;
-            if constexpr (KC) {
-                w = stage[S][b][h];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = xstage[S][b / U][4 * h + e][b % U];
-            }
-            if constexpr (KC && KTAIL && MASK) {
-                const int lim = k_rem - first_k() - 16 * h;
-#pragma unroll
-                for (int d = 1; d < 4; ++d) w[d] = d < lim ? w[d] : 0.0f;
-            }
-            mx[b] = fmaxf(fmaxf(mx[b], fabsf(w[0])), fabsf(w[1]));
-            mx[b] = fmaxf(fmaxf(mx[b], fabsf(w[2])), fabsf(w[3]));
+            const f32x4 w = value<S, MASK>(b, h, k_rem);
 #pragma unroll
             for (int d = 0; d < 2; ++d) {
                 uint32_t q0, q1, q2;
-                split_pair(w[2 * d], w[2 * d + 1], q0, q1, q2);
+                split_pair<false>(w[2 * d], w[2 * d + 1], q0, q1, q2, lost);
                 p[b][0][2 * h + d] = q0; p[b][1][2 * h + d] = q1; p[b][2][2 * h + d] = q2;
             }
         };
@@ -404,18 +458,24 @@ struct DirectOperand {
             for (int t = 0; t < 3; ++t) pc[P][b][t] = __builtin_bit_cast(bf16x8, p[b][t]);
     }
 
+    // The staged tile's part in its rows' statistics.
+    template <int S>
+    __device__ inline void stats(float (&mx)[NROW], uint32_t (&ls)[NROW], int k_rem)
+    {
+        arrange<S>();
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) gather_stats(value<S, true>(b, h, k_rem), mx[b], ls[b]);
+    }
+
     __device__ static inline int map(int b, int i)
     {
         return (b / U) * U * 16 + U * i + (b % U);
     }
-    __device__ static inline int max_row(int tid, int i, int w0) { return w0 + map(i, tid % 16); }
+    __device__ static inline int row_of(int tid, int i, int w0) { return w0 + map(i, tid % 16); }
 };
 
-// Rows (of A) or columns (of B) whose largest magnitude is below this, and not zero, are
-// computed with fp32 MFMAs: bf16 has fp32's exponent range, so a value below
-// 2^-110 loses bits of its third piece, at most 2^-134 in magnitude -- which
-// matters to a row only if the whole row is that small.
-constexpr float kSplitTiny = 7.888609052210118e-31f;  // 2^-100
 // Shorter sums are left to fp32 MFMAs: with few terms the rounding
 // of the result is most of the error, and a split adds its own to it.
 constexpr int kSplitMinK = 32;
@@ -488,56 +548,106 @@ __device__ __forceinline__ void native_pass(const GemmArgs<float>& p, typename M
     }
 }
 
-// Whether the tile has to be computed again with fp32 MFMAs (uniform over the
-// workgroup).  smem: at least 4 * (BM + BN) bytes, no longer in use; *redo: 0.
-template <typename MF, int BM, int BN, int NTHR, typename OpA, typename OpB, int NBM, int NBN>
-__device__ __forceinline__ bool split_failed(const GemmArgs<float>& p, typename MF::acc_t (&acc)[NBM][NBN],
-                            const OpA& opa, const OpB& opb, int m0, int n0, int wm0,
-                            int wn0, int tid, char* smem, int* redo)
+// Whether a tile has to be computed again with fp32 MFMAs.  Two things show
+// that the split did not hold its values:
+// (1) Every infinity and NaN of an operand, every value that rounds to an
+//     infinite bf16 and every overflow leaves a non-finite accumulator (inf * 0
+//     and inf - inf are NaN).
+// (2) A value whose split is inexact (split_pair's lost: it lies below 2^-110)
+//     is held to within 2^-134.  Over K' terms that moves a result by
+//         2^-134 K' (max of its column, if its row holds such a value,
+//                    + max of its row, if its column does),
+//     which is let pass where it is below 2^-24 of the result, as a product's
+//     own dropped terms are.  Tails of a softmax, 2^-120 beside 1, pass; rows
+//     that are tiny as a whole, or whose other values meet zeros, do not.
+// redo_flag: a thread's own view (1, 2: lost bits of the direct, the shared
+// operand; 4: a non-finite accumulator), all that a tile without them pays.
+template <typename MF, int NBM, int NBN>
+__device__ __forceinline__ int redo_flag(const typename MF::acc_t (&acc)[NBM][NBN], uint32_t lost_d,
+                                uint32_t lost_s)
 {
-            // (1) Every infinity and NaN of an operand, every value that rounds
-    // to an infinite bf16 and every overflow leaves a non-finite
-    // accumulator (inf * 0 and inf - inf are NaN): 0 * acc is then not 0.
-    // (2) A row or column that is tiny as a whole (kSplitTiny): a thread
-    // sees part of each row; it raises the flag for its part, and the
-    // whole rows are looked at only then.
-    float z = 0.0f;
+    float z = 0.0f;  // 0 * acc is not 0 where acc is not finite
 #pragma unroll
     for (int i = 0; i < NBM; ++i)
 #pragma unroll
         for (int j = 0; j < NBN; ++j)
 #pragma unroll
             for (int r = 0; r < MF::NACC; ++r) z = fmaf(acc[i][j][r], 0.0f, z);
-    const bool bad = !(z == 0.0f);
-    bool tiny = false;
+    return (z == 0.0f ? 0 : 4) | ((lost_s & kLostBits) != 0 ? 2 : 0) | ((lost_d & kLostBits) != 0 ? 1 : 0);
+}
+
+// redo_fails: a lane's accumulators against (1) and (2): 0, or how many fail
+// (in bits 16 and up; a non-finite one counts as two) over the last one's code.
+// row: largest magnitude of each of the tile's BM rows of A and BN columns of
+// B, as bits; low: not 0 where that row or column holds a value with an inexact
+// split.  terms: K'.
+template <typename MF, typename OpA, typename OpB, int BM, int NBM, int NBN>
+__device__ __forceinline__ int redo_fails(const typename MF::acc_t (&acc)[NBM][NBN], const unsigned* row,
+                                 const unsigned* low, int terms, int wm0, int wn0, int lane)
+{
+    const float unit = 0x1p-110f * (float)terms;  // 2^24 * 2^-134 K'
+    int fails = 0;
 #pragma unroll
-    for (int i = 0; i < OpA::NMAX; ++i) tiny |= opa.mx[i] < kSplitTiny && opa.mx[i] > 0.0f;
+    for (int j = 0; j < NBN; ++j) {
+        const int n = BM + wn0 + OpB::map(j, lane % 16);
+        const float cmax = __builtin_bit_cast(float, row[n]);
+        const bool clow = low[n] != 0;
 #pragma unroll
-    for (int i = 0; i < OpB::NMAX; ++i) tiny |= opb.mx[i] < kSplitTiny && opb.mx[i] > 0.0f;
-    if (bad || tiny) atomicOr(redo, bad ? 2 : 1);
-    __syncthreads();
-    const int flags = __builtin_amdgcn_readfirstlane(*redo);
-    bool native = (flags & 2) != 0;
-    if (flags == 1) {
-        unsigned* row = reinterpret_cast<unsigned*>(smem);  // BM + BN maxima, as bits
-        for (int i = tid; i < BM + BN; i += NTHR) row[i] = 0;
-        __syncthreads();
+        for (int i = 0; i < NBM; ++i)
 #pragma unroll
-        for (int i = 0; i < OpA::NMAX; ++i)
-            atomicMax(row + OpA::max_row(tid, i, wm0), __builtin_bit_cast(unsigned, opa.mx[i]));
-#pragma unroll
-        for (int i = 0; i < OpB::NMAX; ++i)
-            atomicMax(row + BM + OpB::max_row(tid, i, wn0), __builtin_bit_cast(unsigned, opb.mx[i]));
-        __syncthreads();
-        for (int i = tid; i < BM + BN; i += NTHR) {
-            const float m = __builtin_bit_cast(float, row[i]);
-            const bool in = i < BM ? i < p.M - m0 : i - BM < p.N - n0;
-            if (in && m < kSplitTiny && m > 0.0f) atomicOr(redo, 2);
-        }
-        __syncthreads();
-        native = (__builtin_amdgcn_readfirstlane(*redo) & 2) != 0;
+            for (int r = 0; r < MF::NACC; ++r) {
+                const int m = wm0 + OpA::map(i, MF::row(r, lane / 16));
+                const float least = unit * ((low[m] != 0 ? cmax : 0.0f) +
+                                            (clow ? __builtin_bit_cast(float, row[m]) : 0.0f));
+                const float v = fabsf(acc[i][j][r]);
+                const int step = v <= __FLT_MAX__ ? (v >= least ? 0 : 0x10000) : 0x20000;
+                fails = step ? (fails & ~0xffff) + step + ((j * NBM + i) * MF::NACC + r) : fails;
+                // (opaque: otherwise each term is kept until the end, and spills)
+                asm volatile("" : "+v"(fails));
+            }
+        __builtin_amdgcn_sched_barrier(0);
     }
-    return native;
+    return fails;
+}
+
+// A sum of ordinary terms may cancel to nothing (one result in 10^8 at K =
+// 4096): up to kRedoSingles failing results of a wave, one a lane, are
+// looked at by themselves, the wave's lanes taking K between them: such a one
+// passes where 2^-134 per value with an inexact split is below 2^-24 of its sum of magnitudes.
+constexpr int kRedoSingles = 8;
+
+template <typename MF, typename OpA, typename OpB, bool A_KC, bool B_KC, int NBM>
+__device__ __forceinline__ bool redo_needed(const GemmArgs<float>& p, int fails, const float* A, const float* B,
+                                   int m0, int n0, int wm0, int wn0, int k_begin, int k_end, int lane)
+{
+    unsigned long long who = __ballot(fails != 0);
+    if (__ballot(fails >= 0x20000) != 0 || __popcll(who) > kRedoSingles) return true;
+    for (; who != 0; who &= who - 1) {
+        const int src = __ffsll(who) - 1;
+        const int code = __builtin_amdgcn_readlane(fails, src) & 0xffff;
+        const int i = code / MF::NACC % NBM, j = code / MF::NACC / NBM;
+        const int64_t m = m0 + wm0 + OpA::map(i, MF::row(code % MF::NACC, src / 16));
+        const int64_t n = n0 + wn0 + OpB::map(j, src % 16);
+        float sum = 0.0f, loss = 0.0f;
+        if (m < p.M && n < p.N)
+#pragma unroll 1
+            for (int64_t k = k_begin + lane; k < k_end; k += 64) {
+                const float a = A[A_KC ? m * p.lda + k : k * p.lda + m];
+                const float b = B[B_KC ? n * p.ldb + k : k * p.ldb + n];
+                float ma = 0.0f, mb = 0.0f;
+                uint32_t la = 0, lb = 0;
+                gather_stats(f32x4{a, a, a, a}, ma, la);
+                gather_stats(f32x4{b, b, b, b}, mb, lb);
+                sum = fmaf(ma, mb, sum);
+                loss += ((la & kLostBits) != 0 ? mb : 0.0f) + ((lb & kLostBits) != 0 ? ma : 0.0f);
+            }
+        for (int d = 32; d > 0; d >>= 1) {
+            sum += __shfl_xor(sum, d);
+            loss += __shfl_xor(loss, d);
+        }
+        if (!(0x1p-110f * loss <= sum)) return true;
+    }
+    return false;
 }
 
 // BM x BN tile, 32 k per step, WAVES_M x WAVES_N waves, one of them 1; BMC, BNC:
@@ -571,8 +681,9 @@ gemm_split_kernel(GemmArgs<float> p)
     typedef typename std::conditional<A_DIRECT, OpD, OpS>::type OpA;
     typedef typename std::conditional<A_DIRECT, OpS, OpD>::type OpB;
 
-    __shared__ __attribute__((aligned(16))) char smem[2 * OpS::BYTES > 4 * (BM + BN) ? 2 * OpS::BYTES : 4 * (BM + BN)];
+    __shared__ __attribute__((aligned(16))) char smem[2 * OpS::BYTES];
     __shared__ int redo;
+    static_assert(2 * OpS::BYTES >= 8 * (BM + BN), "the rows' statistics lie there after the k loop");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -828,13 +939,74 @@ gemm_split_kernel(GemmArgs<float> p)
                 });
         }
         probe_mark(p, 1);
-        if constexpr (A_DIRECT)
-            native = split_failed<MF, BM, BN, NTHR>(p, acc, opd, ops, m0, n0, wm0, wn0, wave * 64 + lane_id(), smem, &redo);
-        else
-            native = split_failed<MF, BM, BN, NTHR>(p, acc, ops, opd, m0, n0, wm0, wn0, wave * 64 + lane_id(), smem, &redo);
+        // (all waves are past their last use of smem)
+        const int flag = redo_flag<MF>(acc, opd.lost, ops.lost);
+        if (flag) atomicOr(&redo, flag);
+        __syncthreads();
+        const int flags = __builtin_amdgcn_readfirstlane(redo);
+        // Two looks.  The first takes every row of an operand with an inexact
+        // split (be it in what lies beside the matrix) to hold one, and reads the
+        // other operand again for its magnitudes: it lets pass no less than the
+        // second, which reads both.
+        for (int look = (flags & 3) != 0 ? 0 : 1; __builtin_expect(flags != 0, 0) && look < 2; ++look) {
+            const int ln = lane_id(), td = wave * 64 + ln;
+            unsigned* const row = reinterpret_cast<unsigned*>(smem);
+            unsigned* const low = row + BM + BN;
+            const int d0 = A_DIRECT ? 0 : BM, s0 = A_DIRECT ? BM : 0;
+            const bool lost_a = (flags & (A_DIRECT ? 1 : 2)) != 0, lost_b = (flags & (A_DIRECT ? 2 : 1)) != 0;
+            for (int i = td; i < BM + BN; i += NTHR) {
+                row[i] = 0;
+                low[i] = look == 0 && (i < BM ? lost_a : lost_b);
+            }
+            __syncthreads();
+            const bool see_d = look == 0 ? (flags & 2) != 0 : (flags & 3) != 0;
+            const bool see_s = look == 0 ? (flags & 1) != 0 : (flags & 3) != 0;
+            constexpr Int<0> z{};
+            // the next tile's loads run over this one's statistics
+            if (see_d) {
+                float mx[OpD::NROW] = {};
+                uint32_t ls[OpD::NROW] = {};
+                issue_d(z, kt0, kNo);
+                for (kt = kt0; kt < nk; ++kt) {
+                    OpD now = opd;
+                    issue_d(z, kt + 1, kNo);
+                    now.template stats<0>(mx, ls, p.K - kt * BK);
+                }
+#pragma unroll
+                for (int i = 0; i < OpD::NROW; ++i) {
+                    const int x = d0 + OpD::row_of(td, i, w0);
+                    atomicMax(row + x, __builtin_bit_cast(unsigned, mx[i]));
+                    atomicOr(low + x, ls[i] & kLostBits);
+                }
+            }
+            if (see_s) {
+                float mx[OpS::NROW] = {};
+                uint32_t ls[OpS::NROW] = {};
+                issue_s(z, kt0, kNo);
+                for (kt = kt0; kt < nk; ++kt) {
+                    OpS now = ops;
+                    issue_s(z, kt + 1, kNo);
+                    now.template stats<0>(mx, ls, p.K - kt * BK);
+                }
+#pragma unroll
+                for (int i = 0; i < OpS::NROW; ++i) {
+                    const int x = s0 + OpS::row_of(td, i, 0);
+                    atomicMax(row + x, __builtin_bit_cast(unsigned, mx[i]));
+                    atomicOr(low + x, ls[i] & kLostBits);
+                }
+            }
+            __syncthreads();
+            const int fails = redo_fails<MF, OpA, OpB, BM>(acc, row, low, (nk - kt0) * BK, wm0, wn0, ln);
+            if (redo_needed<MF, OpA, OpB, A_KC, B_KC, NBM>(p, fails, A, B, m0, n0, wm0, wn0, kt0 * BK,
+                                                           min(nk * BK, p.K), ln))
+                atomicOr(&redo, 8 << look);
+            __syncthreads();
+            native = (__builtin_amdgcn_readfirstlane(redo) & 8 << look) != 0;
+            if (!native) break;
+        }
     }
     const int lane2 = lane_id();
-    if (native)
+    if (__builtin_expect(native, 0))
         native_pass<MF, OpA, OpB, A_KC, B_KC>(p, acc, A, B, a_org, b_org, a_span, b_span, m0, n0, wm0, wn0,
                                                  kt0 * BK, min(nk * BK, p.K), lane2);
     store_tile<float, MF, OpA, OpB, BM, BN, WTM, WTN, NBM, NBN>(p, acc, t, m0, n0, wm0, wn0, lane2, C);

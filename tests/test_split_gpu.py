@@ -110,3 +110,106 @@ def test_operands_the_split_cannot_hold(cuda, plan, ta, tb):
             # |error| <= 1e-6 of the sum of magnitudes (200 terms); results below
             # 2^-126 are rounded to multiples of 2^-149
             assert (e <= 1e-6 * scale + 2.0 ** -149 * k).all(), (r, float((e / (scale + 1e-300)).max()))
+
+
+ALL_TILES = ["mfma_f32_256x128x16_w4x1", "mfma_f32_128x128x16_w2x2", "mfma_f32_128x128x16_w2x2+splitk3",
+             "mfma_f32_128x128x16_w2x2_o3", "mfma_f32_256x256x32_w4x2", "mfma_f32_256x64x32_w8x1",
+             "mfma_f32_256x48x32_w8x1", "mfma_f32_64x256x32_w1x8", "mfma_f32_48x256x32_w1x8"]
+
+
+def _below_bf16(rng, m, n, k, kind):
+    """Operands whose results rest on values that three bf16 values do not hold."""
+    A = rng.uniform(0.5, 1.0, (m, k))
+    B = rng.uniform(-1.0, 1.0, (k, n))
+    if kind == "graded":        # A D^-1 times D B
+        d = 2.0 ** np.round(np.linspace(0, 124, k))
+        A, B = A / d, B * d[:, None]
+    elif kind == "one":         # one such value a row, against large ones; 1.0 against a zero
+        A[:] = 0.0
+        A[:, 3], A[:, k - 2] = 1.0, 1e-41
+        B[3] = 0.0
+        B[k - 2] *= 1e30
+    elif kind == "single":      # one result of the tile rests on such a value
+        A[:, k - 2], B[:, 9] = 0.0, 0.0
+        A[5, k - 2], B[k - 2, 9] = 1e-41, 1e30
+    elif kind == "identity":    # B's values come through alone, beside an ordinary one a column
+        A[:] = 0.0
+        A[np.arange(min(m, k)), np.arange(min(m, k))] = 1.0
+        B *= 1e-36
+        B[0] = 1.0
+    else:                       # half of each row 2^-e, its ordinary half against zeros
+        A[:, k // 2:] *= 2.0 ** -kind
+        B[:k // 2] = 0.0
+    return A.astype(np.float32), B.astype(np.float32)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("kind", [112, 120, 126, 135, "graded", "one", "single", "identity"])
+def test_values_below_bf16_beside_ordinary_ones(cuda, kind, ta, tb):
+    for i, plan in enumerate(ALL_TILES):
+        m, n, k = {"256x48": (300, 47), "48x256": (40, 300)}.get(plan[9:15], (259, 141)) + (230,)
+        A, B = _below_bf16(np.random.default_rng(SEED + 80 + i), m, n, k, kind)
+        sA, sB = np.ascontiguousarray(A.T if ta else A), np.ascontiguousarray(B.T if tb else B)
+        print(f"{kind} t{ta}{tb} {plan}", flush=True)
+        got = run_sbx(cuda, np.float32, 0, ta, tb, m, n, k, 1.0, sA.ravel(), sA.shape[1], sB.ravel(),
+                      sB.shape[1], 0.0, np.zeros(m * n, np.float32), n, plan=plan)
+        got = got.reshape(m, n).astype(np.float64)
+        A, B = A.astype(np.float64), B.astype(np.float64)
+        # |error| <= 1e-6 of each result's sum of magnitudes (230 terms in fp32), and half of
+        # 2^-149 for each addition of a subnormal result
+        err = np.abs(got - A @ B)
+        assert (err <= 1e-6 * (np.abs(A) @ np.abs(B)) + 2.0 ** -150 * 2 * k).all(), (plan, float(err.max()))
+
+
+@pytest.mark.parametrize("e", [126, 132, 140])
+def test_subnormal_products_of_ordinary_operands(cuda, e):
+    """Products below fp32's normal range: each is rounded to a multiple of 2^-149 and so
+    is each addition, in the six partial products of a term too."""
+    rng = np.random.default_rng(SEED + 95)
+    m, n, k = 257, 130, 256
+    A = (rng.uniform(-1, 1, (m, k)) * 2.0 ** -(e // 2)).astype(np.float32)
+    B = (rng.uniform(-1, 1, (k, n)) * 2.0 ** -(e - e // 2)).astype(np.float32)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    scale = np.abs(A.astype(np.float64)) @ np.abs(B.astype(np.float64))
+    for plan in ALL_TILES[:5]:
+        got = run_sbx(cuda, np.float32, 0, 0, 0, m, n, k, 1.0, A.ravel(), k, B.ravel(), n, 0.0,
+                      np.zeros(m * n, np.float32), n, plan=plan).reshape(m, n)
+        assert (np.abs(got - want) <= 1e-6 * scale + 2.0 ** -150 * 6 * k).all(), plan
+
+
+@pytest.mark.parametrize("upper", [0, 1])
+@pytest.mark.parametrize("trans", [0, 1])
+def test_syrk_operands_the_split_cannot_hold(cuda, upper, trans):
+    import sushiblas_amd as sbx
+    import torch
+    n, k = 400, 300
+    rng = np.random.default_rng(SEED + 97)
+    A = rng.uniform(-1, 1, (n, k)).astype(np.float32)
+    A[150, 7] = np.inf
+    A[260, 200] = np.nan
+    A[33] *= np.float32(1e-36)
+    A[40, 250:] *= np.float32(1e-37)
+    A[40, :250] = 0.0
+    A[41, 250:] *= np.float32(1e20)
+    for plan in ("mfma_f32_128x128x16_w2x2", "mfma_f32_128x128x16_w2x2_o3+splitk2",
+                 "mfma_f32_256x256x32_w4x2"):
+        dA = torch.from_numpy(np.ascontiguousarray(A.T if trans else A)).to(cuda)
+        dC = torch.full((n, n), 5.0, device=cuda)
+        sbx.syrk_ex_plan(sbx.F32, 0, upper, trans, n, k, 1.0, dA, dA.shape[1], 0, 0.0, dC, n, 0, 1, plan)
+        got = dC.cpu().numpy().astype(np.float64)
+        a = A.astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            want = a @ a.T
+            scale = np.abs(a) @ np.abs(a).T
+        want[41, 41] = np.inf  # row 41 times itself, 1.6e41, past fp32's largest
+        i, j = np.indices((n, n))
+        tri = j >= i if upper else j <= i
+        assert (got[~tri] == 5.0).all()
+        fin = tri & np.isfinite(want)
+        np.testing.assert_array_equal(np.isnan(got) & tri, np.isnan(want) & tri)
+        inf = tri & np.isinf(want)
+        np.testing.assert_array_equal(got[inf], want[inf])
+        e = np.abs(got[fin] - want[fin])
+        # fp32 sums in order, the diagonal's of one sign: k roundings of at most 2^-24 of the sum
+        # of magnitudes
+        assert (e <= k * 2.0 ** -24 * scale[fin] + 2.0 ** -150 * 2 * k).all(), plan
