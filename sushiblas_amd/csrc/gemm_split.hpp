@@ -54,7 +54,6 @@ __device__ inline f32x4 split_mma(bf16x8 a, bf16x8 b, f32x4 c)
 // are that lower half.  So the split of every value was exact if and only if
 // the lower half of `lost` is still 0 (checked on the device over all
 // magnitudes from 2^-149 to 2^-90).
-template <bool IN_PLACE>
 __device__ inline void split_pair(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2,
                                   uint32_t& lost)
 {
@@ -72,14 +71,9 @@ __device__ inline void split_pair(float a, float b, uint32_t& p0, uint32_t& p1, 
     const float a1 = a - lo(p0), b1 = b - hi(p0);
     p1 = pack(a1, b1);
     const float a2 = a1 - lo(p1), b2 = b1 - hi(p1);
-    // IN_PLACE: one instruction, where it stands.  As an expression the compiler
-    // keeps a whole tile's remainders to join them at its end: for both
-    // operands that spills, for the direct one alone it is the better schedule
-    // (64 x 65536 x 2048: 114 us in place).
-    if constexpr (IN_PLACE)
-        asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(a2), "v"(b2));
-    else
-        lost |= __builtin_bit_cast(uint32_t, a2) | __builtin_bit_cast(uint32_t, b2);
+    // (one instruction, in place: as an expression the remainders of a whole
+    // tile are kept to be joined at its end, and spill)
+    asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(a2), "v"(b2));
     p2 = pack(a2, b2);
 }
 
@@ -90,8 +84,8 @@ __device__ inline void gather_stats(f32x4 w, float& mx, uint32_t& lost)
 {
     mx = fmaxf(fmaxf(mx, fmaxf(fabsf(w[0]), fabsf(w[1]))), fmaxf(fabsf(w[2]), fabsf(w[3])));
     uint32_t p0, p1, p2;
-    split_pair<true>(w[0], w[1], p0, p1, p2, lost);
-    split_pair<true>(w[2], w[3], p0, p1, p2, lost);
+    split_pair(w[0], w[1], p0, p1, p2, lost);
+    split_pair(w[2], w[3], p0, p1, p2, lost);
 }
 
 // The lane's index, computed anew at each use: what the k loop's tail and the
@@ -257,8 +251,8 @@ struct SplitOperand {
             const f32x4 w = value<S, MASK>(g, u, k_rem);
             u32x2 p[3];
             uint32_t a0, a1, a2, b0, b1, b2;
-            split_pair<true>(w[0], w[1], a0, a1, a2, lost);
-            split_pair<true>(w[2], w[3], b0, b1, b2, lost);
+            split_pair(w[0], w[1], a0, a1, a2, lost);
+            split_pair(w[2], w[3], b0, b1, b2, lost);
             p[0] = u32x2{a0, b0}; p[1] = u32x2{a1, b1}; p[2] = u32x2{a2, b2};
             const int at = KC ? lds0[g % NL] + g / NL * (NL * RSTEP / 16) * BLK
                               : lds0[0] + u * BLK + g * OSTEP * 256;
@@ -436,7 +430,7 @@ struct DirectOperand {
 #pragma unroll
             for (int d = 0; d < 2; ++d) {
                 uint32_t q0, q1, q2;
-                split_pair<false>(w[2 * d], w[2 * d + 1], q0, q1, q2, lost);
+                split_pair(w[2 * d], w[2 * d + 1], q0, q1, q2, lost);
                 p[b][0][2 * h + d] = q0; p[b][1][2 * h + d] = q1; p[b][2][2 * h + d] = q2;
             }
         };
@@ -580,7 +574,9 @@ __device__ __forceinline__ int redo_flag(const typename MF::acc_t (&acc)[NBM][NB
 // (in bits 16 and up; a non-finite one counts as two) over the last one's code.
 // row: largest magnitude of each of the tile's BM rows of A and BN columns of
 // B, as bits; low: not 0 where that row or column holds a value with an inexact
-// split.  terms: K'.
+// split, kOutside where it lies outside C: that comes of the memory beside the
+// operands and counts for nothing.  terms: K'.
+constexpr unsigned kOutside = 1u << 31;
 template <typename MF, typename OpA, typename OpB, int BM, int NBM, int NBN>
 __device__ __forceinline__ int redo_fails(const typename MF::acc_t (&acc)[NBM][NBN], const unsigned* row,
                                  const unsigned* low, int terms, int wm0, int wn0, int lane)
@@ -589,18 +585,20 @@ __device__ __forceinline__ int redo_fails(const typename MF::acc_t (&acc)[NBM][N
     int fails = 0;
 #pragma unroll
     for (int j = 0; j < NBN; ++j) {
-        const int n = BM + wn0 + OpB::map(j, lane % 16);
-        const float cmax = __builtin_bit_cast(float, row[n]);
-        const bool clow = low[n] != 0;
+        const int n = wn0 + OpB::map(j, lane % 16);
+        const float cmax = __builtin_bit_cast(float, row[BM + n]);
+        const unsigned clow = low[BM + n];
 #pragma unroll
         for (int i = 0; i < NBM; ++i)
 #pragma unroll
             for (int r = 0; r < MF::NACC; ++r) {
                 const int m = wm0 + OpA::map(i, MF::row(r, lane / 16));
-                const float least = unit * ((low[m] != 0 ? cmax : 0.0f) +
-                                            (clow ? __builtin_bit_cast(float, row[m]) : 0.0f));
+                const unsigned rlow = low[m];
+                const float least = unit * ((rlow != 0 ? cmax : 0.0f) +
+                                            (clow != 0 ? __builtin_bit_cast(float, row[m]) : 0.0f));
                 const float v = fabsf(acc[i][j][r]);
-                const int step = v <= __FLT_MAX__ ? (v >= least ? 0 : 0x10000) : 0x20000;
+                int step = v <= __FLT_MAX__ ? (v >= least ? 0 : 0x10000) : 0x20000;
+                if ((int)(rlow | clow) < 0) step = 0;
                 fails = step ? (fails & ~0xffff) + step + ((j * NBM + i) * MF::NACC + r) : fails;
                 // (opaque: otherwise each term is kept until the end, and spills)
                 asm volatile("" : "+v"(fails));
@@ -629,18 +627,17 @@ __device__ __forceinline__ bool redo_needed(const GemmArgs<float>& p, int fails,
         const int64_t m = m0 + wm0 + OpA::map(i, MF::row(code % MF::NACC, src / 16));
         const int64_t n = n0 + wn0 + OpB::map(j, src % 16);
         float sum = 0.0f, loss = 0.0f;
-        if (m < p.M && n < p.N)
 #pragma unroll 1
-            for (int64_t k = k_begin + lane; k < k_end; k += 64) {
-                const float a = A[A_KC ? m * p.lda + k : k * p.lda + m];
-                const float b = B[B_KC ? n * p.ldb + k : k * p.ldb + n];
-                float ma = 0.0f, mb = 0.0f;
-                uint32_t la = 0, lb = 0;
-                gather_stats(f32x4{a, a, a, a}, ma, la);
-                gather_stats(f32x4{b, b, b, b}, mb, lb);
-                sum = fmaf(ma, mb, sum);
-                loss += ((la & kLostBits) != 0 ? mb : 0.0f) + ((lb & kLostBits) != 0 ? ma : 0.0f);
-            }
+        for (int64_t k = k_begin + lane; k < k_end; k += 64) {
+            const float a = A[A_KC ? m * p.lda + k : k * p.lda + m];
+            const float b = B[B_KC ? n * p.ldb + k : k * p.ldb + n];
+            float ma = 0.0f, mb = 0.0f;
+            uint32_t la = 0, lb = 0;
+            gather_stats(f32x4{a, a, a, a}, ma, la);
+            gather_stats(f32x4{b, b, b, b}, mb, lb);
+            sum = fmaf(ma, mb, sum);
+            loss += ((la & kLostBits) != 0 ? mb : 0.0f) + ((lb & kLostBits) != 0 ? ma : 0.0f);
+        }
         for (int d = 32; d > 0; d >>= 1) {
             sum += __shfl_xor(sum, d);
             loss += __shfl_xor(loss, d);
@@ -956,7 +953,8 @@ gemm_split_kernel(GemmArgs<float> p)
             const bool lost_a = (flags & (A_DIRECT ? 1 : 2)) != 0, lost_b = (flags & (A_DIRECT ? 2 : 1)) != 0;
             for (int i = td; i < BM + BN; i += NTHR) {
                 row[i] = 0;
-                low[i] = look == 0 && (i < BM ? lost_a : lost_b);
+                const bool inside = i < BM ? i < p.M - m0 : i - BM < p.N - n0;
+                low[i] = !inside ? kOutside : look == 0 && (i < BM ? lost_a : lost_b);
             }
             __syncthreads();
             const bool see_d = look == 0 ? (flags & 2) != 0 : (flags & 3) != 0;

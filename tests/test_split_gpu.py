@@ -213,3 +213,20 @@ def test_syrk_operands_the_split_cannot_hold(cuda, upper, trans):
         # fp32 sums in order, the diagonal's of one sign: k roundings of at most 2^-24 of the sum
         # of magnitudes
         assert (e <= k * 2.0 ** -24 * scale[fin] + 2.0 ** -150 * 2 * k).all(), plan
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("fill", [np.nan, np.inf, 1e-40])
+def test_memory_beside_the_operands_changes_nothing(cuda, fill, ta, tb):
+    """Vector loads of an edge tile bring in the leading dimension's padding:
+    whatever lies there, the result's bits are those of a zero padding."""
+    for i, plan in enumerate(ALL_TILES):
+        m, n, k = {"256x48": (301, 47), "48x256": (41, 301)}.get(plan[9:15], (257, 141)) + (165,)
+        A, lda, B, ldb, C, ldc = make_inputs(np.float32, 0, ta, tb, m, n, k, SEED + 110 + i, pad=(3, 5, 2))
+        got = []
+        for v in (0.0, fill):
+            for X, ld, width in ((A, lda, m if ta else k), (B, ldb, k if tb else n)):
+                X[np.arange(X.size) % ld >= width] = v
+            print(f"{fill} t{ta}{tb} {plan}", flush=True)
+            got.append(run_sbx(cuda, np.float32, 0, ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, plan=plan))
+        np.testing.assert_array_equal(got[0], got[1], plan)
