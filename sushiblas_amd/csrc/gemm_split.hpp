@@ -108,6 +108,19 @@ __device__ __forceinline__ void static_for(F&& f)
     }
 }
 
+// N rows of an x-contiguous operand at one k.  (One is a plain float: an array of one-element
+// vectors ends up in memory.)
+template <int N>
+struct RowVec {
+    typedef float type __attribute__((ext_vector_type(N)));
+    __device__ static inline float get(type x, int u) { return x[u]; }
+};
+template <>
+struct RowVec<1> {
+    typedef float type;
+    __device__ static inline float get(float x, int) { return x; }
+};
+
 // The operand that the waves share: global -> registers -> three bf16 planes
 // in LDS, 32 k at a time.
 //   X: tile extent; NB: its 16-row blocks a wave multiplies (all that are
@@ -152,9 +165,9 @@ struct SplitOperand {
     int row_bytes;  // KC: bytes between sweeps; !KC: between k rows
     int lds0[NL];           // LDS offsets of this thread's first NL groups
     uint32_t lost = 0;      // see split_pair
-    typedef float xvec __attribute__((ext_vector_type(XV)));
+    typedef RowVec<XV> xvec;
     f32x4 stage[KC ? PF : 1][KC ? NG : 1];       // KC: PF tiles in flight, 4 k of a row each
-    xvec xstage[KC ? 1 : PF][KC ? 1 : NG][4];  // !KC: likewise, XV rows at one k each
+    typename xvec::type xstage[KC ? 1 : PF][KC ? 1 : NG][4];  // !KC: likewise, XV rows at one k each
 
     // KC: first k of this thread's vectors
     __device__ static inline int first_k() { return 4 * (lane_id() % VPR); }
@@ -209,12 +222,12 @@ struct SplitOperand {
                     const int so = CHECK ? soff : soff + ro;
                     if constexpr (XV == 4)
                         xstage[S][g][kk] = __builtin_bit_cast(
-                            xvec, __builtin_amdgcn_raw_buffer_load_b128(rs, off, so, CPOL));
+                            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, so, CPOL));
                     else if constexpr (XV == 2)
                         xstage[S][g][kk] = __builtin_bit_cast(
-                            xvec, __builtin_amdgcn_raw_buffer_load_b64(rs, off, so, CPOL));
+                            f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, off, so, CPOL));
                     else
-                        xstage[S][g][kk][0] = __builtin_bit_cast(
+                        xstage[S][g][kk] = __builtin_bit_cast(
                             float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, so, CPOL));
                 }
             }
@@ -232,7 +245,7 @@ struct SplitOperand {
             w = stage[S][g];
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = xstage[S][g][e][u];
+            for (int e = 0; e < 4; ++e) w[e] = xvec::get(xstage[S][g][e], u);
         }
         if constexpr (KC && KTAIL && MASK) {
             const int lim = k_rem - first_k();
@@ -261,15 +274,48 @@ struct SplitOperand {
         }
     }
 
-    // The staged tile's part in its rows' statistics.
+    // The k tile unsplit, for fp32 MFMAs: per 16-row block two halves of 4 octets
+    // of 16 slots of 16 bytes (4 k each), the slots XORed with octet and half so
+    // that 8 consecutive lanes' writes (KC: one row's) and reads meet no bank twice.
+    static constexpr int RAW_BLK = 2048;
+    static_assert((X / 16) * RAW_BLK <= BYTES, "a raw tile takes a split one's place");
     template <int S>
-    __device__ inline void stats(float (&mx)[NROW], uint32_t (&ls)[NROW], int k_rem)
+    __device__ inline void store_raw(char* lds, int tid, int k_rem) const
     {
+        const int x0 = KC ? tid / VPR : chunk(tid) * XV;
+        const int h = KC ? tid / 4 % 2 : (tid >> 3) & 1;
+        const int o0 = KC ? tid % 4 : tid / (2 * XCH);
 #pragma unroll
         for (int g = 0; g < NG; ++g)
 #pragma unroll
-            for (int u = 0; u < XV; ++u)
-                gather_stats(value<S, true>(g, u, k_rem), mx[KC ? g : u], ls[KC ? g : u]);
+            for (int u = 0; u < XV; ++u) {
+                const int x = x0 + (KC ? g * RSTEP : u), o = o0 + (KC ? 0 : g * OSTEP);
+                const int blk = x / (16 * U) * U + x % U, slot = x % (16 * U) / U;
+                *reinterpret_cast<f32x4*>(lds + blk * RAW_BLK + h * 1024 + (o * 16 + (slot ^ (o | 4 * h))) * 16) =
+                    value<S, true>(g, u, k_rem);
+            }
+    }
+    // A lane's fragment of half h in a raw block.
+    __device__ static inline int raw_off(int lane, int h)
+    {
+        const int i = lane % 16, o = lane / 16;
+        return h * 1024 + (o * 16 + (i ^ (o | 4 * h))) * 16;
+    }
+
+    // The staged tile's part in its rows' statistics; next() may stage another.
+    template <int S, typename F>
+    __device__ inline void stats(float (&mx)[NROW], uint32_t (&ls)[NROW], int k_rem, F&& next)
+    {
+        f32x4 w[NG][XV];
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int u = 0; u < XV; ++u) w[g][u] = value<S, true>(g, u, k_rem);
+        next();
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int u = 0; u < XV; ++u) gather_stats(w[g][u], mx[KC ? g : u], ls[KC ? g : u]);
     }
 
     // Tile row of slot i of block b.
@@ -313,9 +359,9 @@ struct DirectOperand {
     static constexpr int NROW = NB;  // rows a lane holds values of
     int voff[KC ? 2 : NW];
     uint32_t lost = 0;  // see split_pair
-    typedef float xvec __attribute__((ext_vector_type(U)));
+    typedef RowVec<U> xvec;
     f32x4 stage[KC ? PF : 1][KC ? NB : 1][2];     // KC: PF tiles in flight
-    xvec xstage[KC ? 1 : PF][KC ? 1 : NW][8];  // !KC: likewise, U rows at one k each
+    typename xvec::type xstage[KC ? 1 : PF][KC ? 1 : NW][8];  // !KC: likewise, U rows at one k each
     bf16x8 pc[NPC][NB][3];
 
     // 4q, and the first k of lane l's KC loads
@@ -369,12 +415,12 @@ struct DirectOperand {
                     const int so = CHECK ? soff : soff + ro;
                     if constexpr (U == 4)
                         xstage[S][w][n] = __builtin_bit_cast(
-                            xvec, __builtin_amdgcn_raw_buffer_load_b128(rs[0], off, so, CPOL));
+                            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs[0], off, so, CPOL));
                     else if constexpr (U == 2)
                         xstage[S][w][n] = __builtin_bit_cast(
-                            xvec, __builtin_amdgcn_raw_buffer_load_b64(rs[0], off, so, CPOL));
+                            f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs[0], off, so, CPOL));
                     else
-                        xstage[S][w][n][0] = __builtin_bit_cast(
+                        xstage[S][w][n] = __builtin_bit_cast(
                             float, __builtin_amdgcn_raw_buffer_load_b32(rs[0], off, so, CPOL));
                 }
         }
@@ -409,7 +455,7 @@ struct DirectOperand {
             w = stage[S][b][h];
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = xstage[S][b / U][4 * h + e][b % U];
+            for (int e = 0; e < 4; ++e) w[e] = xvec::get(xstage[S][b / U][4 * h + e], b % U);
         }
         if constexpr (KC && KTAIL && MASK) {
             const int lim = k_rem - first_k() - 16 * h;
@@ -452,15 +498,21 @@ struct DirectOperand {
             for (int t = 0; t < 3; ++t) pc[P][b][t] = __builtin_bit_cast(bf16x8, p[b][t]);
     }
 
-    // The staged tile's part in its rows' statistics.
-    template <int S>
-    __device__ inline void stats(float (&mx)[NROW], uint32_t (&ls)[NROW], int k_rem)
+    // The staged tile's part in its rows' statistics; next() may stage another.
+    template <int S, typename F>
+    __device__ inline void stats(float (&mx)[NROW], uint32_t (&ls)[NROW], int k_rem, F&& next)
     {
         arrange<S>();
+        f32x4 w[NB][2];
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) gather_stats(value<S, true>(b, h, k_rem), mx[b], ls[b]);
+            for (int h = 0; h < 2; ++h) w[b][h] = value<S, true>(b, h, k_rem);
+        next();
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) gather_stats(w[b][h], mx[b], ls[b]);
     }
 
     __device__ static inline int map(int b, int i)
@@ -471,76 +523,9 @@ struct DirectOperand {
 };
 
 // Shorter sums are left to fp32 MFMAs: with few terms the rounding
-// of the result is most of the error, and a split adds its own to it.
+// of the result is most of the error, and a split adds its own to it.  One k
+// tile holds them.
 constexpr int kSplitMinK = 32;
-
-// Operand reader of the fp32 MFMA pass (native_pass): block b's fragment of
-// the k group at `kg` straight from memory.
-template <typename Op, int NB, bool KC>
-struct NativeRead {
-    __device__ static inline void read(const float* base, int64_t org, int64_t span, int64_t ld,
-                                       int w0, int b0, int x_rem, int kg, int k_end, int lane,
-                                       float (&f)[NB][4])
-    {
-        const int i = lane % 16, q = lane / 16;
-        const int64_t at = org + (KC ? (int64_t)kg : (int64_t)kg * ld);
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc(base + at, span - at * 4);
-        const int k = 4 * q;  // relative to kg
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int x = w0 + Op::map(b0 + b, i);
-            if constexpr (KC) {
-                const int off = x < x_rem && kg + k < k_end ? (int)((x * ld + k) * 4) : kOobOffset;
-                const f32x4 v = __builtin_bit_cast(f32x4, raw_load16(rs, off));
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk) f[b][kk] = kg + k + kk < k_end ? v[kk] : 0.0f;
-            } else {
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    const int off = x < x_rem && kg + k + kk < k_end
-                                        ? (int)(((k + kk) * ld + x) * 4) : kOobOffset;
-                    f[b][kk] = __builtin_bit_cast(
-                        float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
-                }
-            }
-        }
-    }
-};
-
-// acc = the wave's tile over k in [k_begin, k_end) with fp32 MFMAs, operands
-// straight from memory (a cold path: it is kept small, and takes no more registers
-// than the main one).
-template <typename MF, typename OpA, typename OpB, bool A_KC, bool B_KC, int NBM, int NBN>
-__device__ __forceinline__ void native_pass(const GemmArgs<float>& p, typename MF::acc_t (&acc)[NBM][NBN],
-                                   const float* A, const float* B, int64_t a_org, int64_t b_org,
-                                   int64_t a_span, int64_t b_span, int m0, int n0, int wm0, int wn0,
-                                   int k_begin, int k_end, int lane)
-{
-#pragma unroll
-    for (int i = 0; i < NBM; ++i)
-#pragma unroll
-        for (int j = 0; j < NBN; ++j)
-#pragma unroll
-            for (int r = 0; r < MF::NACC; ++r) acc[i][j][r] = 0;
-    for (int kg = k_begin; kg < k_end; kg += MF::Q * 4) {
-        float fa[NBM][4];
-        NativeRead<OpA, NBM, A_KC>::read(A, a_org, a_span, p.lda, wm0, 0, p.M - m0, kg, k_end, lane, fa);
-        constexpr int JC = NBN > 8 ? 8 : NBN;  // blocks of B at a time
-        static_for<0, NBN / JC>([&](auto J) SBX_INLINE {
-            constexpr int j0 = decltype(J)::value * JC;
-            float fb[JC][4];
-            NativeRead<OpB, JC, B_KC>::read(B, b_org, b_span, p.ldb, wn0, j0, p.N - n0, kg, k_end, lane, fb);
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-                for (int i = 0; i < NBM; ++i)
-#pragma unroll
-                    for (int j = 0; j < JC; ++j)
-                        acc[i][j0 + j] = MF::mma(fa[i][kk], fb[j][kk], acc[i][j0 + j]);
-            if constexpr (NBN > JC) __builtin_amdgcn_sched_barrier(0);
-        });
-    }
-}
 
 // Whether a tile has to be computed again with fp32 MFMAs.  Two things show
 // that the split did not hold its values:
@@ -725,179 +710,248 @@ gemm_split_kernel(GemmArgs<float> p)
     const int kt0 = t.is_split ? (int)((int64_t)t.part * nk_all / p.split) : 0;
     const int nk = t.is_split ? (int)((int64_t)(t.part + 1) * nk_all / p.split) : nk_all;
 
-    bool native = p.K < kSplitMinK;
-    if (!native) {
-        OpD opd;
-        OpS ops;
-        opd.init(lane, ld_d, (A_DIRECT ? p.M - m0 : p.N - n0) - w0);
-        ops.init(tid, ld_s, A_DIRECT ? p.N - n0 : p.M - m0);
-        if (tid == 0) redo = 0;
+    OpD opd;
+    OpS ops;
+    // (again after the k loop, whose registers then hold nothing for later)
+    auto init = [&](int ln) SBX_INLINE {
+        opd.init(ln, ld_d, (A_DIRECT ? p.M - m0 : p.N - n0) - w0);
+        ops.init(wave * 64 + ln, ld_s, A_DIRECT ? p.N - n0 : p.M - m0);
+    };
+    init(lane);
+    if (tid == 0) redo = 0;
 
-        // Fixed descriptors for the k tiles that are full and not the last,
-        // moving ones for the rest (as in gemm_mfma_kernel).  A k-contiguous
-        // direct operand takes one descriptor per block of 16 rows.
-        constexpr int ND = D_KC ? NBD : 1;
-        auto d_rsrc = [&](int64_t org, __amdgpu_buffer_rsrc_t (&r)[ND]) SBX_INLINE {
+    // Fixed descriptors for the k tiles that are full and not the last,
+    // moving ones for the rest (as in gemm_mfma_kernel).  A k-contiguous
+    // direct operand takes one descriptor per block of 16 rows.
+    constexpr int ND = D_KC ? NBD : 1;
+    auto d_rsrc = [&](int64_t org, __amdgpu_buffer_rsrc_t (&r)[ND]) SBX_INLINE {
 #pragma unroll
-            for (int b = 0; b < ND; ++b) {
-                const int64_t o = org + (int64_t)OpD::map(b, 0) * ld_d;
-                r[b] = make_rsrc(D + o, d_span - o * 4);
+        for (int b = 0; b < ND; ++b) {
+            const int64_t o = org + (int64_t)OpD::map(b, 0) * ld_d;
+            r[b] = make_rsrc(D + o, d_span - o * 4);
+        }
+    };
+    __amdgpu_buffer_rsrc_t rd0[ND];
+    d_rsrc(d_org, rd0);
+    const __amdgpu_buffer_rsrc_t rs0 = make_rsrc(S + s_org, s_span - s_org * 4);
+    const int d_row_bytes = (int)(ld_d * 4);
+    const int64_t d_tile = D_KC ? (int64_t)NBD * 16 * ld_d + BK : (int64_t)BK * ld_d + NBD * 16;
+    const int64_t s_tile = S_KC ? (int64_t)XS * ld_s + BK : (int64_t)BK * ld_s + XS;
+    const bool fixed_ok = ((int64_t)nk * d_step + d_tile) * 4 < kMaxRecords - 64 &&
+                          ((int64_t)nk * s_step + s_tile) * 4 < kMaxRecords - 64;
+    auto issue_d = [&](auto SET, int kt, auto FIXED) SBX_INLINE {
+        constexpr int st = decltype(SET)::value;
+        if constexpr (decltype(FIXED)::value) {
+            opd.template load<st, false>(rd0, (int)(kt * d_step * 4), d_row_bytes, BK);
+        } else {
+            __amdgpu_buffer_rsrc_t r[ND];
+            d_rsrc(d_org + kt * d_step, r);
+            opd.template load<st, true>(r, 0, d_row_bytes, p.K - kt * BK);
+        }
+    };
+    auto issue_s = [&](auto SET, int kt, auto FIXED) SBX_INLINE {
+        constexpr int st = decltype(SET)::value;
+        if constexpr (decltype(FIXED)::value) {
+            ops.template load<st, false>(rs0, (int)(kt * s_step * 4), BK);
+        } else {
+            const int64_t ps = s_org + kt * s_step;
+            ops.template load<st, true>(make_rsrc(S + ps, s_span - ps * 4), 0, p.K - kt * BK);
+        }
+    };
+    auto commit = [&](auto SET, int kt, int buf, auto MASK) SBX_INLINE {
+#pragma unroll
+        for (int g = 0; g < OpS::NG; ++g)
+            ops.template store<decltype(SET)::value, decltype(MASK)::value>(
+                smem + buf * OpS::BYTES, g, p.K - kt * BK);
+    };
+    // Fragments of one shared block.
+    // JW: shared blocks multiplied side by side, so that the six MFMAs of
+    // one accumulator have others between them.
+    constexpr int JW = PF > 1 && NBD == 1 && NBS % 2 == 0 ? 2 : 1;
+    constexpr int NFS = PF > 1 ? 2 * JW : 1;
+    bf16x8 fs[NFS][3];
+    auto read_s = [&](auto F, int at, int j, int u) SBX_INLINE {
+        fs[decltype(F)::value][u] = *reinterpret_cast<const bf16x8*>(smem + at + j * OpS::BLK + u * OpS::PLANE);
+    };
+    // Products of piece u of a shared block and piece v of the direct
+    // operand's N blocks from i0 on, into their sums t of this k tile (C:
+    // the first, from zero).
+    auto mma = [&](auto P, auto F, auto C, int i0, int u, int v, auto& t) SBX_INLINE {
+        constexpr int pp = decltype(P)::value, f = decltype(F)::value;
+        constexpr int n = (int)(sizeof(t) / sizeof(t[0]));
+        const f32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const f32x4 c = decltype(C)::value ? zero : t[i];
+            if constexpr (A_DIRECT) t[i] = split_mma(opd.pc[pp][i0 + i][v], fs[f][u], c);
+            else t[i] = split_mma(fs[f][u], opd.pc[pp][i0 + i][v], c);
+        }
+    };
+    auto add = [&](int i0, int j, const auto& t) SBX_INLINE {
+        constexpr int n = (int)(sizeof(t) / sizeof(t[0]));
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (A_DIRECT) acc[i0 + i][j][r] += t[i][r];
+                else acc[j][i0 + i][r] += t[i][r];
             }
-        };
-        __amdgpu_buffer_rsrc_t rd0[ND];
-        d_rsrc(d_org, rd0);
-        const __amdgpu_buffer_rsrc_t rs0 = make_rsrc(S + s_org, s_span - s_org * 4);
-        const int d_row_bytes = (int)(ld_d * 4);
-        const int64_t d_tile = D_KC ? (int64_t)NBD * 16 * ld_d + BK : (int64_t)BK * ld_d + NBD * 16;
-        const int64_t s_tile = S_KC ? (int64_t)XS * ld_s + BK : (int64_t)BK * ld_s + XS;
-        const bool fixed_ok = ((int64_t)nk * d_step + d_tile) * 4 < kMaxRecords - 64 &&
-                              ((int64_t)nk * s_step + s_tile) * 4 < kMaxRecords - 64;
-        auto issue_d = [&](auto SET, int kt, auto FIXED) SBX_INLINE {
-            constexpr int st = decltype(SET)::value;
-            if constexpr (decltype(FIXED)::value) {
-                opd.template load<st, false>(rd0, (int)(kt * d_step * 4), d_row_bytes, BK);
-            } else {
-                __amdgpu_buffer_rsrc_t r[ND];
-                d_rsrc(d_org + kt * d_step, r);
-                opd.template load<st, true>(r, 0, d_row_bytes, p.K - kt * BK);
-            }
-        };
-        auto issue_s = [&](auto SET, int kt, auto FIXED) SBX_INLINE {
-            constexpr int st = decltype(SET)::value;
-            if constexpr (decltype(FIXED)::value) {
-                ops.template load<st, false>(rs0, (int)(kt * s_step * 4), BK);
-            } else {
-                const int64_t ps = s_org + kt * s_step;
-                ops.template load<st, true>(make_rsrc(S + ps, s_span - ps * 4), 0, p.K - kt * BK);
-            }
-        };
-        auto commit = [&](auto SET, int kt, int buf, auto MASK) SBX_INLINE {
+    };
+    constexpr bool kTight = NBM * NBN >= 32;  // 128 accumulators: no register to spare
+    // PF == 1 (registers are short): the tile's direct operand is staged,
+    // its shared one in LDS buffer cur.  The next tile's shared loads run
+    // over the first half of the MFMAs, its direct ones over the second.
+    // Piece u of the next shared block is read when this block's MFMAs
+    // have used it.
+    auto step1 = [&](int kt, int cur, auto MASK, auto FIXED) SBX_INLINE {
+        constexpr Int<0> z{};
+        opd.template split<0, 0, decltype(MASK)::value>(p.K - kt * BK);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_s(z, kt + 1, FIXED);
+        __builtin_amdgcn_sched_barrier(0);
+        const int at = cur * OpS::BYTES + OpS::frag_off(kTight ? lane_id() : lane);
 #pragma unroll
-            for (int g = 0; g < OpS::NG; ++g)
-                ops.template store<decltype(SET)::value, decltype(MASK)::value>(
-                    smem + buf * OpS::BYTES, g, p.K - kt * BK);
-        };
-        const int s_off = OpS::frag_off(lane);
-        // Fragments of one shared block.
-        // JW: shared blocks multiplied side by side, so that the six MFMAs of
-        // one accumulator have others between them.
-        constexpr int JW = PF > 1 && NBD == 1 && NBS % 2 == 0 ? 2 : 1;
-        constexpr int NFS = PF > 1 ? 2 * JW : 1;
-        bf16x8 fs[NFS][3];
-        auto read_s = [&](auto F, int buf, int j, int u) SBX_INLINE {
-            fs[decltype(F)::value][u] = *reinterpret_cast<const bf16x8*>(
-                smem + buf * OpS::BYTES + s_off + j * OpS::BLK + u * OpS::PLANE);
-        };
-        // Products of piece u of a shared block and piece v of the direct
-        // operand's N blocks from i0 on, into their sums t of this k tile (C:
-        // the first, from zero).
-        auto mma = [&](auto P, auto F, auto C, int i0, int u, int v, auto& t) SBX_INLINE {
-            constexpr int pp = decltype(P)::value, f = decltype(F)::value;
-            constexpr int n = (int)(sizeof(t) / sizeof(t[0]));
-            const f32x4 zero = {0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < n; ++i) {
-                const f32x4 c = decltype(C)::value ? zero : t[i];
-                if constexpr (A_DIRECT) t[i] = split_mma(opd.pc[pp][i0 + i][v], fs[f][u], c);
-                else t[i] = split_mma(fs[f][u], opd.pc[pp][i0 + i][v], c);
-            }
-        };
-        auto add = [&](int i0, int j, const auto& t) SBX_INLINE {
-            constexpr int n = (int)(sizeof(t) / sizeof(t[0]));
-#pragma unroll
-            for (int i = 0; i < n; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if constexpr (A_DIRECT) acc[i0 + i][j][r] += t[i][r];
-                    else acc[j][i0 + i][r] += t[i][r];
-                }
-        };
-        // PF == 1 (registers are short): the tile's direct operand is staged,
-        // its shared one in LDS buffer cur.  The next tile's shared loads run
-        // over the first half of the MFMAs, its direct ones over the second.
-        // Piece u of the next shared block is read when this block's MFMAs
-        // have used it.
-        auto step1 = [&](int kt, int cur, auto MASK, auto FIXED) SBX_INLINE {
-            constexpr Int<0> z{};
-            opd.template split<0, 0, decltype(MASK)::value>(p.K - kt * BK);
-            __builtin_amdgcn_sched_barrier(0);
-            issue_s(z, kt + 1, FIXED);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 2; u >= 0; --u) read_s(z, cur, 0, u);
-            static_for<0, NBS>([&](auto J) SBX_INLINE {
-                constexpr int j = decltype(J)::value;
-                constexpr int IH = NBD % 2 == 0 ? 2 : 1;  // direct blocks side by side
-                static_for<0, NBD / IH>([&](auto H) SBX_INLINE {
-                    constexpr int i0 = decltype(H)::value * IH;
-                    // the six products: by piece of the shared operand, small ones first
-                    f32x4 t[IH];
-                    static_for<0, 3>([&](auto W) SBX_INLINE {
-                        constexpr int u = 2 - decltype(W)::value;
-                        static_for<0, 3 - u>([&](auto V) SBX_INLINE {
-                            mma(z, z, Int<u == 2>{}, i0, u, 2 - u - decltype(V)::value, t);
-                        });
-                        if constexpr (j + 1 < NBS && i0 + IH == NBD) read_s(z, cur, j + 1, u);
-                    });
-                    add(i0, j, t);
-                    __builtin_amdgcn_sched_barrier(0);
-                });
-                if constexpr (j == NBS / 2 - 1) {
-                    commit(z, kt + 1, cur ^ 1, MASK);
-                    __builtin_amdgcn_sched_barrier(0);
-                    issue_d(z, kt + 1, FIXED);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            });
-            __syncthreads();
-        };
-        // PF > 1: the tile's direct operand is split already (pc[par]), its
-        // shared one in LDS buffer par.  The next tile, in staging set SET, is
-        // split among this tile's MFMAs (the waves of a workgroup run in step:
-        // split first, multiplied then, each unit would wait for the other),
-        // and the set refilled PF tiles on.
-        auto step = [&](auto SET, auto P, int kt, auto MASK, auto FIXED) SBX_INLINE {
-            constexpr int par = decltype(P)::value;
-            static_for<0, JW>([&](auto J) SBX_INLINE {
-#pragma unroll
-                for (int u = 2; u >= 0; --u) read_s(J, par, decltype(J)::value, u);
-            });
-            opd.template split<decltype(SET)::value, par ^ 1, decltype(MASK)::value>(p.K - (kt + 1) * BK);
-            commit(SET, kt + 1, par ^ 1, MASK);
-            issue_s(SET, kt + 1 + PF, FIXED);
-            issue_d(SET, kt + 1 + PF, FIXED);
-            static_for<0, NBS / JW>([&](auto G) SBX_INLINE {
-                constexpr int g = decltype(G)::value, f = g % 2 * JW;
-                if constexpr (g + 1 < NBS / JW)
-                    static_for<0, JW>([&](auto J) SBX_INLINE {
-                        constexpr int jj = decltype(J)::value;
-#pragma unroll
-                        for (int u = 2; u >= 0; --u)
-                            read_s(Int<(g + 1) % 2 * JW + jj>{}, par, (g + 1) * JW + jj, u);
-                    });
-                f32x4 t[JW][NBD];
+        for (int u = 2; u >= 0; --u) read_s(z, at, 0, u);
+        static_for<0, NBS>([&](auto J) SBX_INLINE {
+            constexpr int j = decltype(J)::value;
+            constexpr int IH = NBD % 2 == 0 ? 2 : 1;  // direct blocks side by side
+            static_for<0, NBD / IH>([&](auto H) SBX_INLINE {
+                constexpr int i0 = decltype(H)::value * IH;
+                // the six products: by piece of the shared operand, small ones first
+                f32x4 t[IH];
                 static_for<0, 3>([&](auto W) SBX_INLINE {
                     constexpr int u = 2 - decltype(W)::value;
                     static_for<0, 3 - u>([&](auto V) SBX_INLINE {
-                        static_for<0, JW>([&](auto J) SBX_INLINE {
-                            constexpr int jj = decltype(J)::value;
-                            mma(P, Int<f + jj>{}, Int<u == 2>{}, 0, u, 2 - u - decltype(V)::value, t[jj]);
-                        });
+                        mma(z, z, Int<u == 2>{}, i0, u, 2 - u - decltype(V)::value, t);
+                    });
+                    if constexpr (j + 1 < NBS && i0 + IH == NBD) read_s(z, at, j + 1, u);
+                });
+                add(i0, j, t);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (j == NBS / 2 - 1) {
+                commit(z, kt + 1, cur ^ 1, MASK);
+                __builtin_amdgcn_sched_barrier(0);
+                issue_d(z, kt + 1, FIXED);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
+        __syncthreads();
+    };
+    // PF > 1: the tile's direct operand is split already (pc[par]), its
+    // shared one in LDS buffer par.  The next tile, in staging set SET, is
+    // split among this tile's MFMAs (the waves of a workgroup run in step:
+    // split first, multiplied then, each unit would wait for the other),
+    // and the set refilled PF tiles on.
+    auto step = [&](auto SET, auto P, int kt, auto MASK, auto FIXED) SBX_INLINE {
+        constexpr int par = decltype(P)::value;
+        const int at = par * OpS::BYTES + OpS::frag_off(lane);
+        static_for<0, JW>([&](auto J) SBX_INLINE {
+#pragma unroll
+            for (int u = 2; u >= 0; --u) read_s(J, at, decltype(J)::value, u);
+        });
+        opd.template split<decltype(SET)::value, par ^ 1, decltype(MASK)::value>(p.K - (kt + 1) * BK);
+        commit(SET, kt + 1, par ^ 1, MASK);
+        issue_s(SET, kt + 1 + PF, FIXED);
+        issue_d(SET, kt + 1 + PF, FIXED);
+        static_for<0, NBS / JW>([&](auto G) SBX_INLINE {
+            constexpr int g = decltype(G)::value, f = g % 2 * JW;
+            if constexpr (g + 1 < NBS / JW)
+                static_for<0, JW>([&](auto J) SBX_INLINE {
+                    constexpr int jj = decltype(J)::value;
+#pragma unroll
+                    for (int u = 2; u >= 0; --u)
+                        read_s(Int<(g + 1) % 2 * JW + jj>{}, at, (g + 1) * JW + jj, u);
+                });
+            f32x4 t[JW][NBD];
+            static_for<0, 3>([&](auto W) SBX_INLINE {
+                constexpr int u = 2 - decltype(W)::value;
+                static_for<0, 3 - u>([&](auto V) SBX_INLINE {
+                    static_for<0, JW>([&](auto J) SBX_INLINE {
+                        constexpr int jj = decltype(J)::value;
+                        mma(P, Int<f + jj>{}, Int<u == 2>{}, 0, u, 2 - u - decltype(V)::value, t[jj]);
                     });
                 });
-                static_for<0, JW>([&](auto J) SBX_INLINE { add(0, g * JW + decltype(J)::value, t[decltype(J)::value]); });
             });
-            // Nothing of the next step moves up: its splits would wait for the
-            // youngest loads.  (One block per wave: it may.  There the wave's
-            // own chain of instructions bounds the step, and 1024^3 on 64^2 tiles runs
-            // 21.7 us against 23.6.)
-            if constexpr (NBD > 1) __builtin_amdgcn_sched_barrier(0);
-            __syncthreads();
-            if constexpr (NBD > 1) __builtin_amdgcn_sched_barrier(0);
-        };
+            static_for<0, JW>([&](auto J) SBX_INLINE { add(0, g * JW + decltype(J)::value, t[decltype(J)::value]); });
+        });
+        // Nothing of the next step moves up: its splits would wait for the
+        // youngest loads.  (One block per wave: it may.  There the wave's
+        // own chain of instructions bounds the step, and 1024^3 on 64^2 tiles runs
+        // 21.7 us against 23.6.)
+        if constexpr (NBD > 1) __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        if constexpr (NBD > 1) __builtin_amdgcn_sched_barrier(0);
+    };
 
-        constexpr std::false_type kNo{};
-        constexpr std::true_type kYes{};
+    constexpr std::false_type kNo{};
+    constexpr std::true_type kYes{};
+    // The wave's tile over this unit's k with fp32 MFMAs, in the place of what is
+    // in acc: sums shorter than kSplitMinK from the start (4096^2 x 16 17.5 us,
+    // 1024 x 8192 x 31 12.7; the fp32 MFMA tile kernels 16.5 and 12.4), and tiles
+    // the split cannot hold after it (4096^3 of NaN 1.52 ms, with one infinity
+    // 1.58; those kernels 0.91 and 1.02).  LDS double buffer, one barrier per 32 k.  The next tile's loads run over this one's MFMAs where there are
+    // registers for them; a large tile's MFMAs take 8 us per 32 k, its loads 1.
+    auto fp32_pass = [&]() SBX_INLINE {
+        constexpr Int<0> z{};
+        const int ln = lane_id(), td = wave * 64 + ln;
+        init(ln);
+#pragma unroll
+        for (int i = 0; i < NBM; ++i)
+#pragma unroll
+            for (int j = 0; j < NBN; ++j)
+#pragma unroll
+                for (int r = 0; r < MF::NACC; ++r) acc[i][j][r] = 0;
+        auto issue = [&](int kt) SBX_INLINE {
+            issue_s(z, kt, kNo);
+            issue_d(z, kt, kNo);
+        };
+        if constexpr (!kTight) issue(kt0);
+        int cur = 0;
+#pragma unroll 1
+        for (int kt = kt0; kt < nk; ++kt, cur ^= 1) {
+            const int k_rem = p.K - kt * BK;
+            char* const buf = smem + cur * OpS::BYTES;
+            if constexpr (kTight) issue(kt);
+            ops.template store_raw<0>(buf, td, k_rem);
+            opd.template arrange<0>();
+            f32x4 fd[2][NBD];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < NBD; ++i) fd[h][i] = opd.template value<0, true>(i, h, k_rem);
+            if constexpr (!kTight) issue(kt + 1);
+            __syncthreads();
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (h == 1 && k_rem <= 16) break;
+                const int off = OpS::raw_off(ln, h);
+                constexpr int JW = !kTight && NBS % 2 == 0 ? 2 : 1;  // blocks side by side
+                static_for<0, NBS / JW>([&](auto G) SBX_INLINE {
+                    constexpr int j0 = decltype(G)::value * JW;
+                    f32x4 fs[JW];
+#pragma unroll
+                    for (int j = 0; j < JW; ++j)
+                        fs[j] = *reinterpret_cast<const f32x4*>(buf + off + (j0 + j) * OpS::RAW_BLK);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int j = 0; j < JW; ++j)
+#pragma unroll
+                            for (int i = 0; i < NBD; ++i) {
+                                if constexpr (A_DIRECT)
+                                    acc[i][j0 + j] = MF::mma(fd[h][i][e], fs[j][e], acc[i][j0 + j]);
+                                else
+                                    acc[j0 + j][i] = MF::mma(fs[j][e], fd[h][i][e], acc[j0 + j][i]);
+                            }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            }
+        }
+    };
+
+    bool again = p.K < kSplitMinK;
+    if (!again) {
         // tile t is staged in set (t - kt0) % PF
         static_for<0, PF>([&](auto I) SBX_INLINE {
             issue_s(I, kt0 + decltype(I)::value, kNo);
@@ -947,6 +1001,7 @@ gemm_split_kernel(GemmArgs<float> p)
         // second, which reads both.
         for (int look = (flags & 3) != 0 ? 0 : 1; __builtin_expect(flags != 0, 0) && look < 2; ++look) {
             const int ln = lane_id(), td = wave * 64 + ln;
+            init(ln);
             unsigned* const row = reinterpret_cast<unsigned*>(smem);
             unsigned* const low = row + BM + BN;
             const int d0 = A_DIRECT ? 0 : BM, s0 = A_DIRECT ? BM : 0;
@@ -965,11 +1020,8 @@ gemm_split_kernel(GemmArgs<float> p)
                 float mx[OpD::NROW] = {};
                 uint32_t ls[OpD::NROW] = {};
                 issue_d(z, kt0, kNo);
-                for (kt = kt0; kt < nk; ++kt) {
-                    OpD now = opd;
-                    issue_d(z, kt + 1, kNo);
-                    now.template stats<0>(mx, ls, p.K - kt * BK);
-                }
+                for (kt = kt0; kt < nk; ++kt)
+                    opd.template stats<0>(mx, ls, p.K - kt * BK, [&]() SBX_INLINE { issue_d(z, kt + 1, kNo); });
 #pragma unroll
                 for (int i = 0; i < OpD::NROW; ++i) {
                     const int x = d0 + OpD::row_of(td, i, w0);
@@ -981,11 +1033,8 @@ gemm_split_kernel(GemmArgs<float> p)
                 float mx[OpS::NROW] = {};
                 uint32_t ls[OpS::NROW] = {};
                 issue_s(z, kt0, kNo);
-                for (kt = kt0; kt < nk; ++kt) {
-                    OpS now = ops;
-                    issue_s(z, kt + 1, kNo);
-                    now.template stats<0>(mx, ls, p.K - kt * BK);
-                }
+                for (kt = kt0; kt < nk; ++kt)
+                    ops.template stats<0>(mx, ls, p.K - kt * BK, [&]() SBX_INLINE { issue_s(z, kt + 1, kNo); });
 #pragma unroll
                 for (int i = 0; i < OpS::NROW; ++i) {
                     const int x = s0 + OpS::row_of(td, i, 0);
@@ -999,15 +1048,12 @@ gemm_split_kernel(GemmArgs<float> p)
                                                            min(nk * BK, p.K), ln))
                 atomicOr(&redo, 8 << look);
             __syncthreads();
-            native = (__builtin_amdgcn_readfirstlane(redo) & 8 << look) != 0;
-            if (!native) break;
+            again = (__builtin_amdgcn_readfirstlane(redo) & 8 << look) != 0;
+            if (!again) break;
         }
     }
-    const int lane2 = lane_id();
-    if (__builtin_expect(native, 0))
-        native_pass<MF, OpA, OpB, A_KC, B_KC>(p, acc, A, B, a_org, b_org, a_span, b_span, m0, n0, wm0, wn0,
-                                                 kt0 * BK, min(nk * BK, p.K), lane2);
-    store_tile<float, MF, OpA, OpB, BM, BN, WTM, WTN, NBM, NBN>(p, acc, t, m0, n0, wm0, wn0, lane2, C);
+    if (__builtin_expect(again, 0)) fp32_pass();
+    store_tile<float, MF, OpA, OpB, BM, BN, WTM, WTN, NBM, NBN>(p, acc, t, m0, n0, wm0, wn0, lane_id(), C);
 }
 
 }  // namespace sbx

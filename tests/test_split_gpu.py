@@ -230,3 +230,30 @@ def test_memory_beside_the_operands_changes_nothing(cuda, fill, ta, tb):
             print(f"{fill} t{ta}{tb} {plan}", flush=True)
             got.append(run_sbx(cuda, np.float32, 0, ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, plan=plan))
         np.testing.assert_array_equal(got[0], got[1], plan)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_fp32_pass(cuda, ta, tb):
+    """The tiles' fp32 products: short K, around the 16 and 32 k that its steps
+    take, and longer K with an infinity in each corner of the tiles, whose
+    finite results are fp32 sums in order."""
+    for i, (k, inf) in enumerate([(1, 0), (3, 0), (15, 0), (16, 0), (17, 0), (31, 0), (33, 1), (100, 1), (271, 1)]):
+        for plan in ALL_TILES:
+            if "splitk" in plan and k < 96:
+                continue
+            m, n = {"256x48": (513, 48), "48x256": (48, 513)}.get(plan[9:15], (257, 259))
+            A, lda, B, ldb, C, ldc = make_inputs(np.float32, 0, ta, tb, m, n, k, SEED + 130 + i, pad=(1, 2, 3))
+            if inf:
+                # (flat offsets of op(A)[0, 0] and op(A)[m - 1, k - 1])
+                A[0] = np.inf
+                A[(k - 1) * lda + m - 1 if ta else (m - 1) * lda + k - 1] = -np.inf
+            print(f"fp32 pass {m}x{n}x{k} t{ta}{tb} {plan}", flush=True)
+            got = run_sbx(cuda, np.float32, 0, ta, tb, m, n, k, 1.5, A, lda, B, ldb, 0.5, C, ldc, plan=plan)
+            got = c_window(0, got, m, n, ldc)
+            if inf:
+                assert not np.isfinite(got[0]).any() and not np.isfinite(got[m - 1]).any(), plan
+                A[0] = A[(k - 1) * lda + m - 1 if ta else (m - 1) * lda + k - 1] = 0
+            want = c_window(0, run_oracle(0, ta, tb, m, n, k, 1.5, A, lda, B, ldb, 0.5, C, ldc), m, n, ldc)
+            rows = slice(1, m - 1) if inf else slice(None)
+            err = np.linalg.norm(got[rows].astype(np.float64) - want[rows]) / np.linalg.norm(want[rows])
+            assert err <= TOL[np.float32], (plan, k, err)
