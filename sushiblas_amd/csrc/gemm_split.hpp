@@ -108,6 +108,21 @@ __device__ __forceinline__ void static_for(F&& f)
     }
 }
 
+// Descriptor of an operand whose 32 k rows may span more than 2 GiB (leading
+// dimensions from 2^24 on): offsets and sizes are unsigned.  kOobOffset then
+// no longer lies past its end; a lane that holds rows outside C reads some of the
+// operand instead, and its results are not stored.
+template <bool KC>
+__device__ inline __amdgpu_buffer_rsrc_t operand_rsrc(const float* base, int64_t bytes)
+{
+    constexpr uint32_t most = KC ? (uint32_t)kMaxRecords : 0xfffffff0u;
+    // (32-bit compares: 64-bit ones take vector registers)
+    const int hi = (int)(bytes >> 32);
+    const uint32_t lo = (uint32_t)bytes;
+    const uint32_t n = hi < 0 ? 0 : hi > 0 || lo > most ? most : lo;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)n, kRsrcWord3);
+}
+
 // N rows of an x-contiguous operand at one k.  (One is a plain float: an array of one-element
 // vectors ends up in memory.)
 template <int N>
@@ -217,9 +232,9 @@ struct SplitOperand {
 #pragma unroll
                 for (int kk = 0; kk < 4; ++kk) {
                     // CHECK: as in DirectOperand
-                    const int ro = (g * OSTEP * 4 + kk) * row_bytes;
-                    const int off = CHECK ? voff + ro : voff;
-                    const int so = CHECK ? soff : soff + ro;
+                    const int r = g * OSTEP * 4 + kk;
+                    const int off = CHECK ? (int)((uint32_t)voff + (uint32_t)r * (uint32_t)row_bytes) : voff;
+                    const int so = CHECK ? soff : soff + r * row_bytes;
                     if constexpr (XV == 4)
                         xstage[S][g][kk] = __builtin_bit_cast(
                             f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, so, CPOL));
@@ -410,9 +425,9 @@ struct DirectOperand {
                     const int h = n / 4, e = n % 4;
                     // CHECK: a row past K lies past the descriptor's end (the
                     // row's offset then goes where that is tested for certain)
-                    const int ro = (16 * h + e) * row_bytes;
-                    const int off = CHECK ? voff[w] + ro : voff[w];
-                    const int so = CHECK ? soff : soff + ro;
+                    const int r = 16 * h + e;
+                    const int off = CHECK ? (int)((uint32_t)voff[w] + (uint32_t)r * (uint32_t)row_bytes) : voff[w];
+                    const int so = CHECK ? soff : soff + r * row_bytes;
                     if constexpr (U == 4)
                         xstage[S][w][n] = __builtin_bit_cast(
                             f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs[0], off, so, CPOL));
@@ -728,12 +743,12 @@ gemm_split_kernel(GemmArgs<float> p)
 #pragma unroll
         for (int b = 0; b < ND; ++b) {
             const int64_t o = org + (int64_t)OpD::map(b, 0) * ld_d;
-            r[b] = make_rsrc(D + o, d_span - o * 4);
+            r[b] = operand_rsrc<D_KC>(D + o, d_span - o * 4);
         }
     };
     __amdgpu_buffer_rsrc_t rd0[ND];
     d_rsrc(d_org, rd0);
-    const __amdgpu_buffer_rsrc_t rs0 = make_rsrc(S + s_org, s_span - s_org * 4);
+    const __amdgpu_buffer_rsrc_t rs0 = operand_rsrc<S_KC>(S + s_org, s_span - s_org * 4);
     const int d_row_bytes = (int)(ld_d * 4);
     const int64_t d_tile = D_KC ? (int64_t)NBD * 16 * ld_d + BK : (int64_t)BK * ld_d + NBD * 16;
     const int64_t s_tile = S_KC ? (int64_t)XS * ld_s + BK : (int64_t)BK * ld_s + XS;
@@ -755,7 +770,7 @@ gemm_split_kernel(GemmArgs<float> p)
             ops.template load<st, false>(rs0, (int)(kt * s_step * 4), BK);
         } else {
             const int64_t ps = s_org + kt * s_step;
-            ops.template load<st, true>(make_rsrc(S + ps, s_span - ps * 4), 0, p.K - kt * BK);
+            ops.template load<st, true>(operand_rsrc<S_KC>(S + ps, s_span - ps * 4), 0, p.K - kt * BK);
         }
     };
     auto commit = [&](auto SET, int kt, int buf, auto MASK) SBX_INLINE {

@@ -233,10 +233,10 @@ bool mfma_feasible(const Problem& p, Cfg c)
     if (c == F32_256x48 && p.n > 48) return false;
     if (c == F32_48x256 && p.m > 48) return false;  // and of rows
     const size_t elem = p.dtype == SBX_F32 ? 4 : 8;
-    // (the fp32 tiles whose name says 16 walk 32 k at a time on the bf16 cores)
-    const int bk = p.dtype == SBX_F32 ? 32 : ci.bk;
-    return offsets_fit(!p.ta, ci.bm, bk, p.lda, elem) &&
-           offsets_fit(p.tb, ci.bn, bk, p.ldb, elem) &&
+    // (the fp32 tiles whose name says 16 walk 32 k at a time, with unsigned
+    // offsets into an operand that is not k-contiguous: the same limit)
+    return offsets_fit(!p.ta, ci.bm, ci.bk, p.lda, elem) &&
+           offsets_fit(p.tb, ci.bn, ci.bk, p.ldb, elem) &&
            cdiv(p.m, ci.bm) * cdiv(p.n, ci.bn) < ((int64_t)1 << 31);
 }
 

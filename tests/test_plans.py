@@ -115,3 +115,15 @@ def test_pick_cache_returns_what_the_model_picks():
                                                       ldc, batch)]
                 assert pick in plans, (sh, pick)
             assert pick == first[sh], (rep, sh, pick, first[sh])
+
+
+def test_fp32_tiles_take_leading_dimensions_to_2_25():
+    """An operand that is not k-contiguous: 16 k rows within 2 GiB are enough
+    for the tiles named with a k step of 16, by name and by choice."""
+    most = (0x7ffffff0 - 64 - 4 * 256) // 64 - 1
+    for lda in (1 << 24, most):
+        assert sbx.gemm_select(sbx.F32, 0, 1, 0, 4096, 4096, 64, lda, 4096, 4096) == \
+            "mfma_f32_256x128x16_w4x1"
+        assert sbx.gemm_select(sbx.F32, 0, 1, 0, 2048, 2048, 40, lda, 2048, 2048) == \
+            "mfma_f32_128x128x16_w2x2_o3"
+    assert sbx.gemm_select(sbx.F32, 0, 1, 0, 4096, 4096, 64, 1 << 25, 4096, 4096) == "generic_64x64x16"

@@ -257,3 +257,33 @@ def test_fp32_pass(cuda, ta, tb):
             rows = slice(1, m - 1) if inf else slice(None)
             err = np.linalg.norm(got[rows].astype(np.float64) - want[rows]) / np.linalg.norm(want[rows])
             assert err <= TOL[np.float32], (plan, k, err)
+
+
+@pytest.mark.parametrize("plan", ["mfma_f32_256x128x16_w4x1", "mfma_f32_128x128x16_w2x2_o3",
+                                  "mfma_f32_128x128x16_w2x2+splitk2"])
+@pytest.mark.parametrize("ld", [(1 << 24) + 3, (1 << 25) - 2])
+def test_rows_more_than_2gib_apart_in_a_k_tile(cuda, plan, ld):
+    """Operands whose 32 k rows span 2 to 4 GiB (unsigned buffer offsets): the
+    bits are those of the same values stored densely."""
+    import sushiblas_amd as sbx
+    import torch
+    m, n, k = 259, 131, 71
+    if ld * 16 * 4 + 4 * 256 >= 0x7ffffff0 - 64:
+        ld = (0x7ffffff0 - 64 - 4 * 256) // 64 - 1  # the largest that a 16-k step's offsets allow
+    gen = torch.Generator(device=cuda).manual_seed(SEED)
+    a = torch.empty(k, m, device=cuda).uniform_(-1, 1, generator=gen)
+    b = torch.empty(k, n, device=cuda).uniform_(-1, 1, generator=gen)
+    big = [torch.empty((k - 1) * ld + w, device=cuda) for w in (m, n)]
+    for x, src in zip(big, (a, b)):
+        for r in range(k):
+            x[r * ld:r * ld + src.shape[1]] = src[r]
+    out = []
+    for A, lda, B, ldb in ((a, m, b, n), (big[0], ld, big[1], ld), (a, m, big[1], ld), (big[0], ld, b, n)):
+        C = torch.zeros(m, n, device=cuda)
+        print(f"{plan} lda {lda} ldb {ldb}", flush=True)
+        sbx.gemm_ex_plan(sbx.F32, 0, 1, 0, m, n, k, 1.0, A, lda, 0, B, ldb, 0, 0.0, C, n, 0, 1, plan)
+        out.append(C.cpu().numpy())
+    for o in out[1:]:
+        np.testing.assert_array_equal(o, out[0])
+    want = (a.double().T @ b.double()).cpu().numpy()
+    assert np.linalg.norm(out[0] - want) <= TOL[np.float32] * np.linalg.norm(want)
