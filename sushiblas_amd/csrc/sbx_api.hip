@@ -617,35 +617,40 @@ struct WorkspaceLease {
     ~WorkspaceLease() { release(); }
 };
 
-// The fp32 tiles that are 48 wide and more both ways and 128 one way multiply
-// on the bf16 matrix cores (gemm_split.hpp): 1.1-1.6 times as fast as on the
-// fp32 ones from K = 128 on (8192^3 7.14 -> 4.64 ms; 2048^2 x 128 14.7 -> 12.5
-// us, 65536 x 64 x 512 37.3 -> 31).  The 32-wide tiles, bound by HBM, and the
-// 64-wide ones of 64 and 128 stay on fp32 MFMAs: with one short workgroup per
-// CU the split's longer way from memory to an MFMA has nothing beside it
-// (1024^3 on 64^2 tiles 19.4 us against 21.8, 33870 x 9 x 1420 51.7 against 55.2).
 // Whether an unsplit 256x128 plan, two tiles per CU, runs its tiles in
 // neighbouring pairs, one 8-wave workgroup of 256x256 per CU.  The pair shares
 // each split of B among twice the rows and each wave's split of A among twice
 // the columns: 23 % fewer vector instructions per MFMA, and as the chip's
-// power bounds both, 8192^3 runs 4.37 against 4.69 ms, 4096^3 556 against 591
-// us, 4096^2 x 1024 149.5 against 153.5.  From K = 1024 on (8192^2 x 256 181 against
-// 177 us: one workgroup has no other to overlap its prologue and epilogue
-// with), and where the pairs make no more rounds than the tiles (9000^2 x
-// 3000, 6 rounds against 5: 2378 against 2238 us).
+// power bounds both, 4096^3 runs 573 against 602 us, 8192 x 4096 x 2048 578
+// against 602, 4096^2 x 1024 152 against 158.  From K = 1024 on (8192^2 x 256
+// 181 against 177 us: one workgroup has no other to overlap its prologue and
+// epilogue with); where the pairs make no more rounds than the tiles (9000^2 x
+// 3000, 6 rounds against 5: 2378 against 2238 us); and where the last round
+// holds more tiles than there are CUs: one that holds fewer takes single tiles
+// half the time of pairs (5120 x 4096 x 2048, 128 tiles left: 459 against 529
+// us, 256 left: 474 against 530, 384 left: 574 against 545; after eight rounds,
+// 16640 x 8192 x 4096, 64 left: still 5225 against 5473).
 constexpr int kPairMinK = 1024;
 
 bool tiles_in_pairs(const GemmArgs<float>& a, int nb)
 {
     if (a.split != 1 || a.uplo || a.K < kPairMinK) return false;
     const int64_t cus = cu_count();
+    const int64_t tiles = (int64_t)a.tiles * nb, left = tiles % (2 * cus);
     const int64_t pairs = (int64_t)a.tiles_m * ((a.tiles_n + 1) / 2) * nb;
-    return cdiv(pairs, cus) <= cdiv((int64_t)a.tiles * nb, 2 * cus) &&
+    return (left == 0 || left > cus) && cdiv(pairs, cus) <= cdiv(tiles, 2 * cus) &&
            // the pair's offsets into a k-major B span 256 columns, into a
            // k-contiguous one 256 rows
            offsets_fit(true, 256, 32, a.ldb, 4);
 }
 
+// The tiles of 128x128, 256x64, 64x256 and more multiply on the bf16 matrix
+// cores (gemm_split.hpp): 1.1-1.6 times as fast as on the fp32 ones from K =
+// 128 on (8192^3 7.14 -> 4.58 ms; 2048^2 x 128 14.7 -> 13.7 us, 65536 x 64 x
+// 512 37.3 -> 31).  The 32-wide tiles, bound by HBM, and those of 64x64, 128x64
+// and 64x128 stay on fp32 MFMAs: with one short workgroup per CU the split's
+// longer way from memory to an MFMA has nothing beside it (1024^3 on 64^2
+// tiles 19.4 us against 21.8, 33870 x 9 x 1420 51.7 against 55.2).
 hipError_t launch_cfg(Cfg cfg, GemmArgs<float>& a, bool akc, bool bkc, const Problem& p,
                       int nb, hipStream_t s)
 {

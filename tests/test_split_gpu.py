@@ -287,3 +287,38 @@ def test_rows_more_than_2gib_apart_in_a_k_tile(cuda, plan, ld):
         np.testing.assert_array_equal(o, out[0])
     want = (a.double().T @ b.double()).cpu().numpy()
     assert np.linalg.norm(out[0] - want) <= TOL[np.float32] * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("batch,m,n", [(1, 513, 385), (3, 260, 300), (2, 255, 128)])
+def test_pairs_in_batches_and_with_relu(cuda, batch, m, n, ta, tb):
+    """Unsplit 256x128 plans with K >= 1024 whose few tiles would leave half the CUs
+    idle run singly, in whole or fuller rounds in pairs: both through the batched
+    and the fused entry points, on grids past one round, with ragged edges."""
+    import sushiblas_amd as sbx
+    import torch
+    k = 1056
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tiles = -(-m // 256) * -(-n // 128) * batch
+    # copies of the batch until the last round holds fewer tiles than CUs, or more
+    for want_more in (False, True):
+        reps = next(r for r in range(1, 4 * cus) if (lambda left: left > cus if want_more else 0 < left <= cus)(
+            tiles * r % (2 * cus)))
+        nb = batch * reps
+        gen = torch.Generator(device=cuda).manual_seed(SEED + nb)
+        A = torch.empty((batch, k, m) if ta else (batch, m, k), device=cuda).uniform_(-1, 1, generator=gen)
+        B = torch.empty((batch, n, k) if tb else (batch, k, n), device=cuda).uniform_(-1, 1, generator=gen)
+        A, B = A.repeat(reps, 1, 1), B.repeat(reps, 1, 1)
+        C0 = torch.empty(nb, m, n, device=cuda).uniform_(-1, 1, generator=gen)
+        want = (A[:batch].mT if ta else A[:batch]).double().contiguous() @ (
+            (B[:batch].mT if tb else B[:batch]).double().contiguous())
+        args = (sbx.F32, 0, ta, tb, m, n, k, 1.5, A, A.shape[2], A[0].numel(), B, B.shape[2], B[0].numel(),
+                0.5)
+        C, R = C0.clone(), C0.clone()
+        print(f"{nb} x {m}x{n}x{k} t{ta}{tb}: {tiles * reps} tiles", flush=True)
+        sbx.gemm_ex_plan(*args, C, n, m * n, nb, "mfma_f32_256x128x16_w4x1")
+        sbx.gemm_fused(*args, R, n, m * n, nb)
+        for z in range(0, nb, max(1, nb // 7)):
+            w = 1.5 * want[z % batch] + 0.5 * C0[z].double()
+            for got, ref in ((C[z], w), (R[z], w.clamp_min(0))):
+                assert (got - ref).norm() <= TOL[np.float32] * ref.norm(), (nb, z)
