@@ -779,12 +779,7 @@ gemm_split_kernel(GemmArgs<float> p)
             ops.template store<decltype(SET)::value, decltype(MASK)::value>(
                 smem + buf * OpS::BYTES, g, p.K - kt * BK);
     };
-    // Fragments of one shared block.
-    // JW: shared blocks multiplied side by side, so that the six MFMAs of
-    // one accumulator have others between them.
-    constexpr int JW = PF > 1 && NBD == 1 && NBS % 2 == 0 ? 2 : 1;
-    constexpr int NFS = PF > 1 ? 2 * JW : 1;
-    bf16x8 fs[NFS][3];
+    bf16x8 fs[PF][3];  // fragments of one shared block (PF > 1: and of the next)
     auto read_s = [&](auto F, int at, int j, int u) SBX_INLINE {
         fs[decltype(F)::value][u] = *reinterpret_cast<const bf16x8*>(smem + at + j * OpS::BLK + u * OpS::PLANE);
     };
@@ -813,6 +808,7 @@ gemm_split_kernel(GemmArgs<float> p)
             }
     };
     constexpr bool kTight = NBM * NBN >= 32;  // 128 accumulators: no register to spare
+    static_assert(NBD % 2 == 0 && PF <= 2, "direct blocks are multiplied two side by side");
     // PF == 1 (registers are short): the tile's direct operand is staged,
     // its shared one in LDS buffer cur.  The next tile's shared loads run
     // over the first half of the MFMAs, its direct ones over the second.
@@ -829,17 +825,16 @@ gemm_split_kernel(GemmArgs<float> p)
         for (int u = 2; u >= 0; --u) read_s(z, at, 0, u);
         static_for<0, NBS>([&](auto J) SBX_INLINE {
             constexpr int j = decltype(J)::value;
-            constexpr int IH = NBD % 2 == 0 ? 2 : 1;  // direct blocks side by side
-            static_for<0, NBD / IH>([&](auto H) SBX_INLINE {
-                constexpr int i0 = decltype(H)::value * IH;
+            static_for<0, NBD / 2>([&](auto H) SBX_INLINE {
+                constexpr int i0 = decltype(H)::value * 2;
                 // the six products: by piece of the shared operand, small ones first
-                f32x4 t[IH];
+                f32x4 t[2];
                 static_for<0, 3>([&](auto W) SBX_INLINE {
                     constexpr int u = 2 - decltype(W)::value;
                     static_for<0, 3 - u>([&](auto V) SBX_INLINE {
                         mma(z, z, Int<u == 2>{}, i0, u, 2 - u - decltype(V)::value, t);
                     });
-                    if constexpr (j + 1 < NBS && i0 + IH == NBD) read_s(z, at, j + 1, u);
+                    if constexpr (j + 1 < NBS && i0 + 2 == NBD) read_s(z, at, j + 1, u);
                 });
                 add(i0, j, t);
                 __builtin_amdgcn_sched_barrier(0);
@@ -861,42 +856,31 @@ gemm_split_kernel(GemmArgs<float> p)
     auto step = [&](auto SET, auto P, int kt, auto MASK, auto FIXED) SBX_INLINE {
         constexpr int par = decltype(P)::value;
         const int at = par * OpS::BYTES + OpS::frag_off(lane);
-        static_for<0, JW>([&](auto J) SBX_INLINE {
 #pragma unroll
-            for (int u = 2; u >= 0; --u) read_s(J, at, decltype(J)::value, u);
-        });
+        for (int u = 2; u >= 0; --u) read_s(Int<0>{}, at, 0, u);
         opd.template split<decltype(SET)::value, par ^ 1, decltype(MASK)::value>(p.K - (kt + 1) * BK);
         commit(SET, kt + 1, par ^ 1, MASK);
         issue_s(SET, kt + 1 + PF, FIXED);
         issue_d(SET, kt + 1 + PF, FIXED);
-        static_for<0, NBS / JW>([&](auto G) SBX_INLINE {
-            constexpr int g = decltype(G)::value, f = g % 2 * JW;
-            if constexpr (g + 1 < NBS / JW)
-                static_for<0, JW>([&](auto J) SBX_INLINE {
-                    constexpr int jj = decltype(J)::value;
+        static_for<0, NBS>([&](auto J) SBX_INLINE {
+            constexpr int j = decltype(J)::value, f = j % 2;
+            if constexpr (j + 1 < NBS)
 #pragma unroll
-                    for (int u = 2; u >= 0; --u)
-                        read_s(Int<(g + 1) % 2 * JW + jj>{}, at, (g + 1) * JW + jj, u);
-                });
-            f32x4 t[JW][NBD];
+                for (int u = 2; u >= 0; --u) read_s(Int<(j + 1) % 2>{}, at, j + 1, u);
+            f32x4 t[NBD];
             static_for<0, 3>([&](auto W) SBX_INLINE {
                 constexpr int u = 2 - decltype(W)::value;
                 static_for<0, 3 - u>([&](auto V) SBX_INLINE {
-                    static_for<0, JW>([&](auto J) SBX_INLINE {
-                        constexpr int jj = decltype(J)::value;
-                        mma(P, Int<f + jj>{}, Int<u == 2>{}, 0, u, 2 - u - decltype(V)::value, t[jj]);
-                    });
+                    mma(P, Int<f>{}, Int<u == 2>{}, 0, u, 2 - u - decltype(V)::value, t);
                 });
             });
-            static_for<0, JW>([&](auto J) SBX_INLINE { add(0, g * JW + decltype(J)::value, t[decltype(J)::value]); });
+            add(0, j, t);
         });
         // Nothing of the next step moves up: its splits would wait for the
-        // youngest loads.  (One block per wave: it may.  There the wave's
-        // own chain of instructions bounds the step, and 1024^3 on 64^2 tiles runs
-        // 21.7 us against 23.6.)
-        if constexpr (NBD > 1) __builtin_amdgcn_sched_barrier(0);
+        // youngest loads.
+        __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
-        if constexpr (NBD > 1) __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_barrier(0);
     };
 
     constexpr std::false_type kNo{};
@@ -990,18 +974,17 @@ gemm_split_kernel(GemmArgs<float> p)
                 for (; kt + 1 < nk - 1; ++kt, cur ^= 1) step1(kt, cur, kNo, kYes);
             for (; kt < nk; ++kt, cur ^= 1) step1(kt, cur, kYes, kNo);
         } else {
-            constexpr int UN = PF == 3 ? 6 : PF == 2 ? 2 : 4;
             // every tile a step loads (up to kt + 1 + PF) is full and not the last
             if (fixed_ok)
-                for (; kt + UN + PF < nk - 1; kt += UN)
-                    static_for<0, UN>([&](auto I) SBX_INLINE {
+                for (; kt + 2 + PF < nk - 1; kt += 2)
+                    static_for<0, 2>([&](auto I) SBX_INLINE {
                         constexpr int i = decltype(I)::value;
-                        step(Int<(i + 1) % PF>{}, Int<(i & 1)>{}, kt + i, kNo, kYes);
+                        step(Int<(i + 1) % PF>{}, Int<i>{}, kt + i, kNo, kYes);
                     });
-            for (; kt < nk; kt += UN)
-                static_for<0, UN>([&](auto I) SBX_INLINE {
+            for (; kt < nk; kt += 2)
+                static_for<0, 2>([&](auto I) SBX_INLINE {
                     constexpr int i = decltype(I)::value;
-                    if (kt + i < nk) step(Int<(i + 1) % PF>{}, Int<(i & 1)>{}, kt + i, kYes, kNo);
+                    if (kt + i < nk) step(Int<(i + 1) % PF>{}, Int<i>{}, kt + i, kYes, kNo);
                 });
         }
         probe_mark(p, 1);

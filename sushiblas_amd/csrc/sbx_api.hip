@@ -173,14 +173,14 @@ int candidate_cfgs(int dtype, int64_t m, int64_t n, int uplo, int64_t cus, Cfg* 
         out[c++] = wide;
         if (f32) out[c++] = F32_64x64;
     } else if (f32 && cdiv(m, 256) * cdiv(n, 256) >= cus * 3 / 4) {
-        // Large fp32.  Two 256x128 workgroups per CU (64x128 per wave)
-        // overlap each other's prologue and epilogue; they beat the 256^2
-        // tile, which runs alone on its CU, on all 15 shapes timed (8192^3
-        // 7211 vs 7277 us, 12288 x 8192 x 1024 1405 vs 1468 us), so the
-        // 256^2 tile is left to SYRK.  They lead where their grid is (nearly)
+        // Large fp32.  Two 256x128 workgroups per CU overlap each other's
+        // prologue and epilogue; where the 256^2 tile is the faster one,
+        // tiles_in_pairs puts two of them into one, so it is a candidate of
+        // its own for SYRK only.  They lead where their grid is (nearly)
         // whole rounds; elsewhere the 128^2 tile at two per CU, whose finer
         // grid and split tail land closer to whole rounds, comes first
-        // (5000^2 x 1000: 376 against 422 us, 5120^3: 1786 against 1872 us).
+        // (measured on the fp32 MFMA tiles that these plans were before:
+        // 5000^2 x 1000: 376 against 422 us, 5120^3: 1786 against 1872 us).
         *large = true;
         const int64_t slots = 2 * cus, left = cdiv(m, 256) * cdiv(n, 128) % slots;
         const bool whole = left == 0 || left >= slots * 7 / 8;
@@ -272,8 +272,13 @@ int check_ld(int layout, bool trans, int64_t rows, int64_t cols, int64_t ld)
 //     (partial bytes the reduction reads) / W, and each part kPartSec;
 //   * the one-launch small-problem kernel is modelled on its own (see
 //     small_seconds).
+// The fp32 tiles that now multiply on the bf16 matrix cores (launch_cfg) keep
+// the constants of the fp32 MFMA tiles they were fitted on: from K = 128 on
+// they run 1.1-1.6 times as fast as modelled, cut into ranges of one or two of
+// their 32-k steps up to 13 % slower than those did (SYRK n = 520, k = 197:
+// 13.0 against 11.4 us).
 // Whole rounds run unsplit; only the tail (T mod P*CUs tiles, or all of them)
-// may be cut into s k-ranges of at least two k tiles each, s from kSplitSet;
+// may be cut into s k-ranges of at least two k tiles of the name's each, s from kSplitSet;
 // a split is taken if predicted >= 0.5 % faster than the fewer ranges before it.
 // Split partials live in a workspace cached per (device, stream): calls on
 // one stream are ordered, so they can share it; the first call that needs
@@ -397,7 +402,8 @@ constexpr double kSmallBwBatch = 7.1474e+12;
 // The split-K space of a tile config: whole rounds run unsplit, and the
 // `rem` tiles of the tail (every tile of every entry, for a batch whose grid
 // fills less than one round) may be cut into 2 .. smax k-ranges of at least
-// two k tiles each.  smax == 0: no split (the small-problem and generic
+// two k tiles each, as the plan's name counts them (a plan named with 16 that
+// steps 32 k may get one step a range).  smax == 0: no split (the small-problem and generic
 // kernels, fewer than four k tiles, a batch that fills a round, no tail).
 // Entry z's partials follow entry z-1's, so the workspace holds one launch's
 // entries (zmax).
@@ -975,10 +981,10 @@ int run(const Problem& p, T alpha, T beta, int algo, hipStream_t stream, Cfg* ch
             a.tiles_m = (int)cdiv(p.m, ci.bm);
             a.tiles_n = (int)cdiv(p.n, ci.bn);
             // GROUP_M: the height of the tile-column walk.  An XCD's 64
-            // resident 256x128 workgroups then cover 4 x 16 tiles (1024 rows
-            // of A, 2048 columns of B), which fetches 2.3 GB from beyond L2
-            // at 8192^3 against 3.4 GB for 8 x 8, in the same time.  The
-            // fp64 128^2 tile likewise: 12.9 GB from beyond L2 at 8192^3
+            // resident 256x128 workgroups cover 4 x 16 tiles (1024 rows of A,
+            // 2048 columns of B; 4.6 GB read from beyond L2 at 8192^3), its
+            // 32 of 256x256 (tiles_in_pairs) 8 x 4 (2048 rows, 1024 columns;
+            // 3.8 GB).  The fp64 128^2 tile likewise: 12.9 GB from beyond L2 at 8192^3
             // against 13.5 GB for 8 (19.3 for 2, 22.6 for 16), same time;
             // its SYRK 9.1 against 9.4 GB.
             const int gm = cfg == F32_256x128 || cfg == F64_128x128 ? 4 : 8;
