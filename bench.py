@@ -146,7 +146,7 @@ PROBE_BLOCKS = 4096  # workgroups per dispatch whose stamps are kept
 PROBE_POINTS = 4  # stamp points per workgroup (SBX_PROBE_POINTS)
 
 
-def probe_summary(t, ndisp, flops, dtype, call_ms, khz, cus):
+def probe_summary(t, ndisp, flops, dtype, call_ms, khz, cus, kernel=""):
     """Clock, loop span and MFMA busy of the timed dispatches, from the probe
     build's per-workgroup stamps (see sushiblas_amd/csrc/sbx_probe.h).
 
@@ -160,7 +160,8 @@ def probe_summary(t, ndisp, flops, dtype, call_ms, khz, cus):
     import numpy as np
     if khz <= 0 or ndisp <= 0:
         return None
-    per_clk = (256 if dtype == "f32" else 128) * cus  # dense MFMA flop per cycle, MI355X
+    # dense MFMA flop per cycle, MI355X; on the bf16 cores (4096) six products for one of fp32
+    per_clk = (4096 / 6 if any(x in kernel for x in SPLIT_TILES) else 256 if dtype == "f32" else 128) * cus
     t = np.asarray(t).reshape(-1, PROBE_BLOCKS, PROBE_POINTS, 2).astype(np.float64)
     rows = []
     for d in range(min(ndisp, t.shape[0])):
@@ -200,7 +201,7 @@ def probe_summary(t, ndisp, flops, dtype, call_ms, khz, cus):
 def time_launches(fn, steps, warmup, min_warm_s=0.0, probe=None):
     """Average device time per call of fn() over `steps` back-to-back calls,
     measured with HIP events on the stream the kernels run on.  With --probe
-    and a dict `probe` = {"flops": F, "dtype": "f32"|"f64"}, the timed
+    and a dict `probe` = {"flops": F, "dtype": "f32"|"f64"[, "kernel": plan]}, the timed
     dispatches' stamps are recorded and probe["out"] gets probe_summary().
 
     `warmup` untimed calls come first; with min_warm_s > 0, more untimed calls
@@ -240,7 +241,8 @@ def time_launches(fn, steps, warmup, min_warm_s=0.0, probe=None):
         sbx.probe_set(None, 0, 0)
         probe["out"] = probe_summary(stamps.cpu().numpy().view(np.uint64), ndisp, probe["flops"],
                                      probe["dtype"], ms, sbx.probe_wall_clock_khz(),
-                                     torch.cuda.get_device_properties(0).multi_processor_count)
+                                     torch.cuda.get_device_properties(0).multi_processor_count,
+                                     probe.get("kernel", ""))
         del stamps
     return ms  # ms
 
@@ -442,7 +444,7 @@ def run_config(dtype, layout, ta, tb, m, n, k, alpha, beta, seed, steps, warmup,
         torch.cuda.synchronize()
         host = host + (C.cpu().numpy(),)
     flops = 2.0 * m * n * k
-    probe = {"flops": flops, "dtype": dtype}
+    probe = {"flops": flops, "dtype": dtype, "kernel": name}
     ms = time_launches(step, steps, warmup, min_warm_s=0.25, probe=probe)
     tflops = flops / (ms * 1e-3) / 1e12
     nbytes = (m * k + k * n + m * n * (2 if beta != 0 else 1)) * A.element_size()
@@ -946,7 +948,7 @@ def main():
         sbx.sgemm(0, 0, 0, m, n, k, alpha, A, k, B, n, beta, C, n)
 
     flops = 2.0 * m * n * k
-    probe = {"flops": flops, "dtype": "f32"}
+    probe = {"flops": flops, "dtype": "f32", "kernel": kernel}
     ms = time_launches(step, args.steps, args.warmup, probe=probe)
     value = flops / (ms * 1e-3) / 1e12
     traffic = read_traffic("headline")

@@ -4,7 +4,7 @@
 // An fp32 value x of 2^-110 and above is the exact sum of three bf16 values (8
 // significant bits each, rounded to nearest): x = x0 + x1 + x2 with
 // |x1| <= 2^-8 |x0| and |x2| <= 2^-17 |x0|.  (Below that it is one if its last
-// bit is 2^-133 or more, bf16's smallest value; see redo_needed for the
+// bit is 2^-133 or more, bf16's smallest value; see redo_flag for the
 // others.)  A product of two such sums has nine terms; the six largest,
 //     a2 b0 + a0 b2 + a1 b1 + a1 b0 + a0 b1 + a0 b0,
 // leave out less than 2^-24 of |a b|.  Each is one bf16 MFMA; the six of a 32-k
@@ -17,11 +17,12 @@
 // chain by 1.5e-6.)
 //   Error of K-term dot products against 64-bit sums, 2-norm, fp32 MFMA
 // chain -> this sum (256 x 256, uniform on [-1, 1) / on [0, 1) / normal):
+//     K = 32     1.0e-7 / 8.4e-8 / 1.0e-7  ->  3.6e-8 / 3.4e-8 / 3.8e-8
 //     K = 512    4.1e-7 / 3.1e-7 / 4.1e-7  ->  8.6e-8 / 6.0e-8 / 8.9e-8
 //     K = 8192   1.6e-6 / 1.2e-6 / 1.6e-6  ->  3.0e-7 / 2.1e-7 / 3.1e-7
 //   The bf16 MFMAs run at 16 times the fp32 ones' rate (2.5 PFLOP/s against
 // 157 TFLOP/s), so six of them per product take 3/8 of the time; what the chip
-// holds of that is bound by its power (the clock falls to 1.75 GHz), so work
+// holds of that is bound by its power (the clock falls to 1.8-2.0 GHz), so work
 // beside the MFMAs (LDS traffic, the split itself) is what the layout below
 // saves.
 #pragma once
@@ -47,7 +48,7 @@ __device__ inline f32x4 split_mma(bf16x8 a, bf16x8 b, f32x4 c)
 
 // Two fp32 values -> their three bf16 pieces, packed (first value in the low
 // half).  The differences are exact.  An infinity, or a value that rounds to
-// one, leaves NaNs (see redo_needed).
+// one, leaves NaNs (see redo_flag).
 // lost: gathers the last remainders' bits.  A remainder of 2^-126 and more has 8
 // significant bits and none in its word's lower half; a smaller one is a
 // multiple of 2^-149 whose bits below 2^-133, those that bf16 has no place for,

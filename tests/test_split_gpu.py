@@ -2,8 +2,8 @@
 (gemm_split.hpp): each tile by name at sizes around its edges, K tails and
 every transpose against the oracle accumulating in double; an error no larger
 than fp32 sums in order leave; and the operands the split cannot hold
-(infinities, NaN, values past bf16's largest, rows and columns below 2^-100),
-which the kernel computes again with fp32 MFMAs."""
+(infinities, NaN, values past bf16's largest, values below 2^-110 that a
+result rests on), for which the kernel computes the tile again with fp32 MFMAs."""
 import numpy as np
 import pytest
 
@@ -83,7 +83,9 @@ def test_operands_the_split_cannot_hold(cuda, plan, ta, tb):
     opa[20, :] *= np.float32(1e-36)      # a row below 2^-100: pieces would lose bits
     opa[21, :] = 0.0
     opb[:, 9] *= np.float32(1e-34)
-    opa[30, 40] = np.float32(1e-36)      # one tiny value in an ordinary row
+    # one tiny value in an ordinary row (the bound below is the row's: results that rest on
+    # such a value are test_values_below_bf16_beside_ordinary_ones')
+    opa[30, 40] = np.float32(1e-36)
     got = run_sbx(cuda, np.float32, 0, ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, ldc, plan=plan)
     got = c_window(0, got, m, n, ldc).astype(np.float64)
     with np.errstate(invalid="ignore", over="ignore"):
